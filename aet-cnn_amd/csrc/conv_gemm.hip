@@ -27,13 +27,12 @@
 // compile-time constant.  Workgroups are remapped so that neighbouring
 // tiles of one K slice (M-tiles sharing an input patch, N-tiles sharing a
 // delta slice) run on the same XCD and share its L2.
-#include "common.hpp"
+#include "conv_split.hpp"
 
 #include <type_traits>
 
 namespace ach {
 
-typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v32f __attribute__((ext_vector_type(32)));
 
 constexpr int GNT = 256;     // threads per workgroup
@@ -48,50 +47,11 @@ constexpr int LDP = 4;       // LDS row padding (floats)
 // ds_read2st64 reads it without address arithmetic.  Their stores write whole
 // 64-lane row segments (no conflicts).
 constexpr int LDP_FWD = 0;
-constexpr unsigned kOOB = 0x80000000u;  // buffer offset that reads as 0
 constexpr int WGRAD_BK = 16;            // k-tile of the weight-gradient GEMM
 // weight-gradient workgroups aimed for (tiles x splits) in the (image,
 // position) K order
 constexpr int WGRAD_TARGET = 2048;
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, unsigned bytes)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes,
-                                             0x00020000);
-}
-
-// element offset -> byte offset, or the out-of-range offset when invalid
-__device__ __forceinline__ int boff(bool ok, int elem)
-{
-    return ok ? elem * 4 : (int)kOOB;
-}
-
-// the builtin returns the loaded dword as an integer: reinterpret its bits
-__device__ __forceinline__ float bload(__amdgpu_buffer_rsrc_t r, int byte_off)
-{
-    return __int_as_float((int)__builtin_amdgcn_raw_buffer_load_b32(r, byte_off, 0, 0));
-}
-
-// The same with a wave-uniform byte offset in the instruction's scalar
-// offset operand (an SGPR): loaders with loop-invariant per-thread offsets
-// add the k-tile's uniform advance there instead of in one VGPR per load.
-// Callers keep voff + soff inside the buffer for every in-range voff (the
-// prefetch past the last k-tile re-reads the last tile), so the address is
-// valid whether or not the range check includes the scalar offset; an
-// out-of-range voff (>= 2^31) reads zero either way.
-__device__ __forceinline__ float bload_so(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff)
-{
-    return __int_as_float(
-        (int)__builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
-}
-
-
-struct ConvGeom {
-    int B, C, H, W;    // input
-    int F, KS, S, P;   // filters, kernel, stride, pad
-    int OH, OW;
-    FastDiv dkk, dks;  // division by KS*KS and by KS
-};
 
 // ===========================================================================
 // Operand loaders.  Each provides, for its k-tile width BK:
@@ -140,20 +100,6 @@ struct AWeightsT {
 // f = tid + 256*i of the BK x BM tile (row f / (BM/4), columns 4*(f % (BM/4))
 // .. +3), one dwordx4 buffer load and one 16-byte LDS store each, instead of
 // four dword loads and stores.
-__device__ __forceinline__ float4 bload4(__amdgpu_buffer_rsrc_t r, int byte_off)
-{
-    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, byte_off, 0, 0);
-    return make_float4(__int_as_float((int)v[0]), __int_as_float((int)v[1]),
-                       __int_as_float((int)v[2]), __int_as_float((int)v[3]));
-}
-
-__device__ __forceinline__ float4 bload4_so(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff)
-{
-    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0);
-    return make_float4(__int_as_float((int)v[0]), __int_as_float((int)v[1]),
-                       __int_as_float((int)v[2]), __int_as_float((int)v[3]));
-}
-
 template <int BM, int BK>
 struct AWeightsT4 {
     static constexpr bool SPILL = BK == 18;
@@ -933,31 +879,6 @@ struct PlainOperand {
 
 // ===========================================================================
 // Problems: operand loaders + k range + epilogue.
-// ===========================================================================
-// Output epilogue of the forward GEMMs: the layer's bias and activation
-// applied to each finished sum, as the separate passes would apply them
-// (IOData.addBias then activate, IOData.c:43-72), in one branch-free form
-// so the kernel keeps a single epilogue.  Kernels instantiated with the
-// epilogue (EPI) hold every accumulator in VGPRs at the end; tiles of at
-// most 128 rows keep that within their occupancy.
-//   v += bias[m]            (no bias: v + -0.0f, which is v for every v)
-//   v = v > 0 ? v : (float)(slope * (double)v)
-// slope 0.1 is act_forward's leaky; slope 0 gives relu's v * (v > 0)
-// (+-0 with the sign of v, NaN kept); slope 1 is linear.  The default
-// (no bias, slope 1) leaves v unchanged.  The logistic activation, with
-// its double exp, stays a separate pass.
-struct Epi {
-    const float *bias = nullptr;
-    double slope = 1.0;
-    bool active() const { return bias != nullptr || slope != 1.0; }
-    __device__ __forceinline__ float apply(float v, int m) const
-    {
-        const float b = bias ? bias[m] : -0.0f;
-        v = v + b;
-        return v > 0.f ? v : (float)(slope * (double)v);
-    }
-};
-
 // Forward: y[b][m][p] = sum_k Wt[k][m] * im2col(x)[k][b*OHW+p].  With
 // splits > 1 each z-slice of K writes part[z][m][n] and a fixed-order
 // reduction produces y (used when the tile grid alone cannot fill the GPU).
@@ -2757,11 +2678,22 @@ static FwdPlan fwd_plan(const ConvGeom &g, bool kg_ok = true)
     return pl;
 }
 
-static size_t fwd_part_bytes(const ConvGeom &g, bool kg_ok = true)
+// bytes of partial sums: of the fp32 plan, which a call needs, and the most
+// that a call makes use of (the workspace queries)
+static size_t fp32_part_bytes(const ConvGeom &g, bool kg_ok = true)
 {
     const FwdPlan pl = fwd_plan(g, kg_ok);
     if (pl.pslices() <= 1) return 0;
     return (size_t)pl.pslices() * g.F * g.B * g.OH * g.OW * sizeof(float);
+}
+static size_t fwd_part_bytes(const ConvGeom &g, bool kg_ok = true)
+{
+    const FwdPlan pl = fwd_plan(g, kg_ok);
+    const SplitFwdPlan sp = split_fwd_plan(g, kg_ok, pl.pslices(), 1 << 30);
+    const size_t need = fp32_part_bytes(g, kg_ok);
+    if (!sp.ok || sp.splits <= 1) return need;
+    const size_t n = (size_t)sp.splits * g.F * g.B * g.OH * g.OW * sizeof(float);
+    return n > need ? n : need;
 }
 
 // EPI: the bias / activation epilogue in the GEMM (used without a K split
@@ -2878,29 +2810,38 @@ static int fwd_bm_padded(const ConvGeom &g, const FwdPlan &pl, const float *x, c
     return launch_gemm(p, M, N, pl.splits, st);
 }
 
-// w: k-major filter Wt[K][M]; part: fwd_part_bytes(g) of scratch (or NULL
-// when no split is planned).  An active epilogue e runs in the GEMM when K
+// w: k-major filter Wt[K][M]; part: part_bytes of scratch, at least
+// fp32_part_bytes(g).  pieces: the three-piece bf16 kernel (conv_split.hip)
+// may run.  An active epilogue e runs in the GEMM when K
 // is not split, or in the split-K reduction.
 // w_nat: a fully connected geometry's w is the filter itself (W[F][K]).
 static int fwd_impl(const ConvGeom &g, const float *x, const float *w, float *y, float *part,
-                    hipStream_t st, const Epi &e = Epi(), bool w_nat = false, bool kg_ok = true)
+                    size_t part_bytes, hipStream_t st, const Epi &e = Epi(), bool w_nat = false, bool kg_ok = true,
+                    bool pieces = true)
 {
     if (fwd_small_k(g))
         return e.active() ? fwd_small_k_launch<true>(g, x, w, y, e, w_nat, st)
                           : fwd_small_k_launch<false>(g, x, w, y, e, w_nat, st);
     const FwdPlan pl = fwd_plan(g, kg_ok);
-    const bool unsplit = pl.pslices() == 1;  // no partial sums
-    const int ps = pl.pslices();
+    const size_t room = part ? part_bytes / ((size_t)g.F * g.B * g.OH * g.OW * sizeof(float)) : 0;
+    SplitFwdPlan sp = split_fwd_plan(g, kg_ok, pl.pslices(), room > 1024 ? 1024 : (int)room);
+    sp.ok = sp.ok && pieces;
+    const int ps = sp.ok ? sp.splits : pl.pslices();
+    const bool unsplit = ps == 1;  // no partial sums
     const bool gemm_epi = e.active() && unsplit;
     int rc;
-    if (gemm_epi) {
+    if (sp.ok) {
+        rc = split_fwd_launch(g, sp, x, w, y, part, e, st);
+        if (rc || unsplit) return rc;
+    } else if (gemm_epi) {
         if (pl.bm == 32) rc = fwd_bm<32, true>(g, pl, x, w, y, part, e, w_nat, st);
         else if (pl.bm == 96) rc = fwd_bm_padded<96, true>(g, pl, x, w, y, part, e, st);
         else if (pl.bm == 64) rc = fwd_bm<64, true>(g, pl, x, w, y, part, e, w_nat, st);
         else rc = fwd_bm<128, true>(g, pl, x, w, y, part, e, w_nat, st);
         return rc;
     }
-    if (pl.bm == 32) rc = fwd_bm<32, false>(g, pl, x, w, y, part, e, w_nat, st);
+    if (sp.ok) rc = ACH_OK;
+    else if (pl.bm == 32) rc = fwd_bm<32, false>(g, pl, x, w, y, part, e, w_nat, st);
     else if (pl.bm == 96) rc = fwd_bm_padded<96, false>(g, pl, x, w, y, part, e, st);
     else if (pl.bm == 64) rc = fwd_bm<64, false>(g, pl, x, w, y, part, e, w_nat, st);
     else rc = fwd_bm<128, false>(g, pl, x, w, y, part, e, w_nat, st);
@@ -3243,10 +3184,11 @@ int ach_conv_fwd(const ach_conv_desc *d, const float *x, const float *w, float *
     hipStream_t st = as_stream(stream);
     const int M = g.F, K = g.C * g.KS * g.KS;
     float *wt = (float *)ws;
-    float *part = (float *)((char *)ws + align256((size_t)M * K * sizeof(float)));
+    const size_t fb = align256((size_t)M * K * sizeof(float));
+    float *part = (float *)((char *)ws + fb);
     // a fully connected geometry reads the filter in its own layout, and so
     // does the patch-staged shallow-im2col kernel
-    if (fc_geom(g)) return fwd_impl(g, x, w, y, part, st, Epi(), true);
+    if (fc_geom(g)) return fwd_impl(g, x, w, y, part, ws_bytes - fb, st, Epi(), true);
     if (fwd_small_k(g)) {
         const int rc0 = fwd_small_k_launch<false>(g, x, w, y, Epi(), true, st);
         if (rc0 != ACH_EUNSUPPORTED) return rc0;
@@ -3255,7 +3197,7 @@ int ach_conv_fwd(const ach_conv_desc *d, const float *x, const float *w, float *
                        wt, M, K);
     int rc = check_launch();
     if (rc) return rc;
-    return fwd_impl(g, x, wt, y, part, st);
+    return fwd_impl(g, x, wt, y, part, ws_bytes - fb, st);
 }
 
 // geometry of stride-1 dgrad seen as a forward convolution of dy
@@ -3293,15 +3235,18 @@ int ach_conv_bwd_data(const ach_conv_desc *d, const float *dy, const float *w, f
     if (!xy && dgrad_small_c(g) && !fc_geom(g)) return dgrad_small_c_launch(g, dy, w, dx, st);
     if (!xy && g.S == 1 && g.P <= g.KS - 1) {
         const size_t tot = (size_t)g.F * g.C * g.KS * g.KS;
-        float *part = (float *)((char *)ws + align256(tot * sizeof(float)));
+        const size_t fb = align256(tot * sizeof(float));
+        float *part = (float *)((char *)ws + fb);
         // 1x1: the flipped k-major filter Wft[f][c] is W itself
-        if (g.KS == 1) return fwd_impl(dgrad_as_fwd(g), dy, w, dx, part, st, Epi(), false, false);
+        if (g.KS == 1) 
+            return fwd_impl(dgrad_as_fwd(g), dy, w, dx, part, ws_bytes - fb, st, Epi(), false,
+                            false);
         float *wf = (float *)ws;
         hipLaunchKernelGGL(k_weights_flip_kmajor, dim3(grid_for(tot, 256)), dim3(256), 0, st, w,
                            wf, g.F, g.C, g.KS * g.KS);
         int rc = check_launch();
         if (rc) return rc;
-        return fwd_impl(dgrad_as_fwd(g), dy, wf, dx, part, st, Epi(), false, false);
+        return fwd_impl(dgrad_as_fwd(g), dy, wf, dx, part, ws_bytes - fb, st, Epi(), false, false);
     }
     // Strided convolution (unequal strides included): the reference's
     // per-image TN GEMM + col2im (ConvolutionalLayer.c:933-945).  Not on any
@@ -3365,9 +3310,9 @@ int ach_conv_fwd_prepared(const ach_conv_desc *d, const float *x, const float *w
     if (!fits_int(d)) return ACH_EUNSUPPORTED;
     if (conv_xy(d)) return xy_fwd(d, x, wt, true, y, ws, ws_bytes, stream);
     const ConvGeom g = geom(d);
-    const size_t need = fwd_part_bytes(g);
+    const size_t need = fp32_part_bytes(g);
     if (need && (!ws || ws_bytes < need)) return ACH_EWORKSPACE;
-    return fwd_impl(g, x, wt, y, (float *)ws, as_stream(stream), Epi(), fc_geom(g));
+    return fwd_impl(g, x, wt, y, (float *)ws, ws_bytes, as_stream(stream), Epi(), fc_geom(g));
 }
 
 int ach_conv_is_fully_connected(const ach_conv_desc *d)
@@ -3375,9 +3320,9 @@ int ach_conv_is_fully_connected(const ach_conv_desc *d)
     return conv_ok(d) && fc_geom(geom(d)) ? 1 : 0;
 }
 
-int ach_conv_fwd_bias_act_prepared(const ach_conv_desc *d, const float *x, const float *wt,
-                                   const float *bias, int activation, float *y, void *ws,
-                                   size_t ws_bytes, ach_stream_t stream)
+static int fwd_bias_act(const ach_conv_desc *d, const float *x, const float *wt,
+                        const float *bias, int activation, float *y, void *ws, size_t ws_bytes,
+                        ach_stream_t stream, bool pieces)
 {
     if (!conv_ok(d) || !x || !wt || !y) return ACH_EINVAL;
     if (activation != ACH_LOGISTIC && activation != ACH_RELU && activation != ACH_LINEAR &&
@@ -3391,16 +3336,31 @@ int ach_conv_fwd_bias_act_prepared(const ach_conv_desc *d, const float *x, const
         if (rc) return rc;
         return ach_activate(y, (size_t)g.B * g.F * g.OH * g.OW, activation, stream);
     }
-    const size_t need = fwd_part_bytes(g);
+    const size_t need = fp32_part_bytes(g);
     if (need && (!ws || ws_bytes < need)) return ACH_EWORKSPACE;
     Epi e;
     e.bias = bias;
     e.slope = activation == ACH_LEAKY ? 0.1 : (activation == ACH_RELU ? 0.0 : 1.0);
     hipStream_t st = as_stream(stream);
-    const int rc = fwd_impl(g, x, wt, y, (float *)ws, st, e, fc_geom(g));
+    const int rc = fwd_impl(g, x, wt, y, (float *)ws, ws_bytes, st, e, fc_geom(g), true,
+                            pieces);
     // logistic, with its double exp, runs after the bias epilogue
     if (rc || activation != ACH_LOGISTIC) return rc;
     return ach_activate(y, (size_t)g.B * g.F * g.OH * g.OW, activation, stream);
+}
+
+int ach_conv_fwd_bias_act_prepared(const ach_conv_desc *d, const float *x, const float *wt,
+                                   const float *bias, int activation, float *y, void *ws,
+                                   size_t ws_bytes, ach_stream_t stream)
+{
+    return fwd_bias_act(d, x, wt, bias, activation, y, ws, ws_bytes, stream, true);
+}
+
+int ach_conv_fwd_train_prepared(const ach_conv_desc *d, const float *x, const float *wt,
+                                const float *bias, int activation, float *y, void *ws,
+                                size_t ws_bytes, ach_stream_t stream)
+{
+    return fwd_bias_act(d, x, wt, bias, activation, y, ws, ws_bytes, stream, false);
 }
 
 int ach_conv_bwd_data_prepared(const ach_conv_desc *d, const float *dy, const float *w,
@@ -3415,10 +3375,10 @@ int ach_conv_bwd_data_prepared(const ach_conv_desc *d, const float *dy, const fl
     if (dgrad_small_c(g) && !fc_geom(g)) return dgrad_small_c_launch(g, dy, w, dx, as_stream(stream));
     if (g.KS > 1 && !wft) return ACH_EINVAL;
     const ConvGeom t = dgrad_as_fwd(g);
-    const size_t need = fwd_part_bytes(t, false);
+    const size_t need = fp32_part_bytes(t, false);
     if (need && (!ws || ws_bytes < need)) return ACH_EWORKSPACE;
-    return fwd_impl(t, dy, g.KS == 1 ? w : wft, dx, (float *)ws, as_stream(stream), Epi(), false,
-                    false);
+    return fwd_impl(t, dy, g.KS == 1 ? w : wft, dx, (float *)ws, ws_bytes, as_stream(stream),
+                    Epi(), false, false);
 }
 
 size_t ach_conv_bwd_filter_workspace(const ach_conv_desc *d)

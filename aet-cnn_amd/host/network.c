@@ -183,6 +183,16 @@ static ach_conv_desc conv_desc(const an_layer *l)
 
 static int fusable(int act) { return act == ACH_LEAKY || act == ACH_RELU || act == ACH_LINEAR; }
 
+/* the forward GEMM (with bias and activation) into out: a training step's
+ * form or the inference one                                                */
+static int forward_sums(const ach_conv_desc *d, an_state st, const an_layer *l,
+                        const float *biases, int activation, float *out, ach_stream_t s)
+{
+    return (st.train ? ach_conv_fwd_train_prepared : ach_conv_fwd_bias_act_prepared)(
+        d, st.input, l->weights_kmajor, biases, activation, out, st.workspace,
+        st.workspace_bytes, s);
+}
+
 static int conv_forward(an_network *net, an_layer *l, an_state st)
 {
     ach_conv_desc d = conv_desc(l);
@@ -190,8 +200,7 @@ static int conv_forward(an_network *net, an_layer *l, an_state st)
     ach_stream_t s = net->stream;
     if (l->batch_normalize) {
         /* conv output goes straight into NormData.x; BN writes output */
-        AN_CHECK(ach_conv_fwd_prepared(&d, st.input, l->weights_kmajor, l->x, st.workspace,
-                                       st.workspace_bytes, s));
+        AN_CHECK(forward_sums(&d, st, l, NULL, ACH_LINEAR, l->x, s));
         const int act = fusable(l->activation) ? l->activation : ACH_LINEAR;
         if (st.train)
             AN_CHECK(ach_bn_train_fwd_from_x(l->x, l->output, l->batch, l->n, spatial,
@@ -207,11 +216,8 @@ static int conv_forward(an_network *net, an_layer *l, an_state st)
     }
     /* conv + addBias + activate in one pass (the GEMM epilogue) */
     if (fusable(l->activation) || l->activation == ACH_LOGISTIC)
-        return ach_conv_fwd_bias_act_prepared(&d, st.input, l->weights_kmajor, l->biases,
-                                              l->activation, l->output, st.workspace,
-                                              st.workspace_bytes, s);
-    AN_CHECK(ach_conv_fwd_prepared(&d, st.input, l->weights_kmajor, l->output, st.workspace,
-                                   st.workspace_bytes, s));
+        return forward_sums(&d, st, l, l->biases, l->activation, l->output, s);
+    AN_CHECK(forward_sums(&d, st, l, NULL, ACH_LINEAR, l->output, s));
     AN_CHECK(ach_add_bias(l->output, l->biases, l->batch, l->n, spatial, s));
     return ach_activate(l->output, (size_t)l->batch * l->outputs, l->activation, s);
 }

@@ -180,6 +180,14 @@ int ach_conv_fwd_prepared(const ach_conv_desc *d, const float *x, const float *w
 int ach_conv_fwd_bias_act_prepared(const ach_conv_desc *d, const float *x, const float *wt,
                                    const float *bias, int activation, float *y, void *ws,
                                    size_t ws_bytes, ach_stream_t stream);
+/* The same for a training step's forward: every sum on the fp32 matrix
+ * instructions, so that a step's sums -- whose last bits decide branches of
+ * activations and argmaxes of pools, which later steps amplify -- do not
+ * depend on the rounding of the faster forms the other forward calls may
+ * take.  bias NULL and ACH_LINEAR: ach_conv_fwd_prepared's form.           */
+int ach_conv_fwd_train_prepared(const ach_conv_desc *d, const float *x, const float *wt,
+                                const float *bias, int activation, float *y, void *ws,
+                                size_t ws_bytes, ach_stream_t stream);
 /* stride-1 only (ACH_EUNSUPPORTED otherwise); w is read for 1x1 filters,
  * wft otherwise                                                             */
 int ach_conv_bwd_data_prepared(const ach_conv_desc *d, const float *dy, const float *w,

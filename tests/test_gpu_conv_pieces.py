@@ -1,0 +1,96 @@
+"""The convolution kernels that take every float as three bf16 pieces
+(conv_split.hip): forward and input gradient against 64-bit references where
+their tiles, channel chunks and K parts end, and infinities and NaNs.
+
+Bound, per output: the six piece products kept of a*b leave out less than
+2^-24 |ab|, and a matrix instruction adds 16 products with one rounding, so
+with K' = k*k*ceil(C/16) instructions (and a few more additions for K parts)
+|error| <= (K' + 8) 2^-24 sum |a||b|."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import aetcnn
+import refs64
+from aetcnn import DeviceArray as D, check
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    # (B, C, H, W, F, k, p)
+    (1, 16, 8, 16, 32, 3, 1),      # one tile, one chunk, one wave of filters
+    (2, 17, 5, 5, 1, 3, 1),        # ragged chunk of one channel, one filter, images in a tile
+    (3, 31, 9, 7, 33, 3, 1),       # 33 filters: two waves along M, ragged N
+    (2, 48, 13, 13, 65, 3, 1),     # 65 filters: three waves, three chunks
+    (1, 47, 37, 29, 97, 3, 1),     # 97 filters: four waves
+    (2, 64, 16, 16, 130, 3, 1),    # M tiles of 128 with a ragged second
+    (1, 32, 6, 64, 40, 3, 1),      # two rows of 64 per tile
+    (1, 16, 3, 130, 24, 3, 1),     # rows wider than a tile
+    (3, 24, 4, 4, 20, 3, 0),       # no padding: the input gradient pads by 2
+    (2, 32, 7, 6, 48, 3, 2),       # padding 2
+    (9, 40, 8, 8, 16, 3, 1),       # two images per tile, odd batch
+    (5, 20, 9, 9, 30, 5, 2),       # 5x5
+    (2, 33, 27, 27, 96, 5, 2),     # 5x5 on odd planes: one LDS buffer
+    (2, 16, 8, 8, 16, 5, 0),       # 5x5 without padding
+    (64, 128, 8, 8, 128, 3, 1),    # K parts as two groups of a workgroup and slices
+    (128, 96, 13, 13, 256, 3, 1),  # K slices of a grid between one and two rounds
+]
+
+
+def bound(absref, k, c):
+    return (k * k * -(-c // 16) + 8) * 2.0 ** -24 * absref
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_forward_and_input_gradient(gpu, shape):
+    B, Cc, H, W, F, k, p = shape
+    rng = np.random.default_rng(sum(shape))
+    x = rng.standard_normal((B, Cc, H, W)).astype(np.float32)
+    w = rng.standard_normal((F, Cc, k, k)).astype(np.float32)
+    oh, ow = H + 2 * p - k + 1, W + 2 * p - k + 1
+    dy = rng.standard_normal((B, F, oh, ow)).astype(np.float32)
+    d = aetcnn.ConvDesc(B, Cc, H, W, F, k, 1, p)
+    nb = max(gpu.ach_conv_fwd_workspace(C.byref(d)), gpu.ach_conv_bwd_data_workspace(C.byref(d)))
+    ws, dx_, dw, ddy = D(nb // 4 + 64), D.from_numpy(x), D.from_numpy(w), D.from_numpy(dy)
+    y, dx = D(dy.shape), D(x.shape)
+    check(gpu.ach_conv_fwd(C.byref(d), dx_.ptr, dw.ptr, y.ptr, ws.ptr, nb, None))
+    check(gpu.ach_conv_bwd_data(C.byref(d), ddy.ptr, dw.ptr, dx.ptr, ws.ptr, nb, None))
+    ref, mag = refs64.conv_ref(x, w, 1, p), refs64.conv_ref(abs(x), abs(w), 1, p)
+    assert np.all(abs(y.numpy() - ref) <= bound(mag, k, Cc))
+    ref = refs64.dgrad_ref(dy, w, x.shape, 1, p)
+    mag = refs64.dgrad_ref(abs(dy), abs(w), x.shape, 1, p)
+    assert np.all(abs(dx.numpy() - ref) <= bound(mag, k, F))
+
+
+@pytest.mark.parametrize("shape", [(2, 32, 9, 9, 48, 3, 1), (64, 128, 8, 8, 128, 3, 1)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, np.float32(3.4e38)])
+def test_non_finite_and_largest_values(gpu, shape, value):
+    """A non-finite (or just finite) input or weight gives what fp32
+    arithmetic gives: the outputs of the fp32 form of the same call agree in
+    their infinities and NaNs, and elsewhere to rounding."""
+    B, Cc, H, W, F, k, p = shape
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((B, Cc, H, W)).astype(np.float32)
+    w = rng.standard_normal((F, Cc, k, k)).astype(np.float32)
+    x[0, 3, 4, 4] = value
+    w[7, 1, 0, 2] = value if abs(value) > 3.39e38 else 1.0
+    d = aetcnn.ConvDesc(B, Cc, H, W, F, k, 1, p)
+    nb = gpu.ach_conv_fwd_workspace(C.byref(d))
+    ws, dx, dw = D(nb // 4 + 64), D.from_numpy(x), D.from_numpy(w)
+    wt = D(w.size)
+    job = aetcnn.FilterJob(d, dw.ptr, wt.ptr, None)
+    check(gpu.ach_conv_prepare_filters(1, C.byref(job), None))
+    a, b = D((B, F, H, W)), D((B, F, H, W))
+    check(gpu.ach_conv_fwd_prepared(C.byref(d), dx.ptr, wt.ptr, a.ptr, ws.ptr, nb, None))
+    check(gpu.ach_conv_fwd_train_prepared(C.byref(d), dx.ptr, wt.ptr, None, aetcnn.LINEAR, b.ptr,
+                                          ws.ptr, nb, None))
+    a, b = a.numpy().astype(np.float64), b.numpy().astype(np.float64)
+    fin = np.isfinite(b)
+    assert not fin.all() and fin.any()
+    assert np.array_equal(np.isnan(a), np.isnan(b))
+    assert np.array_equal(a[np.isinf(b)], b[np.isinf(b)])
+    near = fin & (abs(b) < 1e30)  # sums without the large value
+    assert np.all(abs(a[near] - b[near]) <= 1e-5 * abs(b[near]).max())
+    assert np.all(abs(a[fin] - b[fin]) <= 1e-5 * abs(b[fin]) + 1e-5 * abs(b[near]).max())
