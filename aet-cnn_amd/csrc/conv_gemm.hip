@@ -28,6 +28,7 @@
 // tiles of one K slice (M-tiles sharing an input patch, N-tiles sharing a
 // delta slice) run on the same XCD and share its L2.
 #include "conv_split.hpp"
+#include "conv_wsplit.hpp"
 
 #include <type_traits>
 
@@ -3178,13 +3179,13 @@ int ach_conv_fwd(const ach_conv_desc *d, const float *x, const float *w, float *
 {
     if (!conv_ok(d) || !x || !w || !y) return ACH_EINVAL;
     if (!fits_int(d)) return ACH_EUNSUPPORTED;
-    if (!ws || ws_bytes < ach_conv_fwd_workspace(d)) return ACH_EWORKSPACE;
     if (conv_xy(d)) return xy_fwd(d, x, w, false, y, ws, ws_bytes, stream);
     const ConvGeom g = geom(d);
     hipStream_t st = as_stream(stream);
     const int M = g.F, K = g.C * g.KS * g.KS;
     float *wt = (float *)ws;
     const size_t fb = align256((size_t)M * K * sizeof(float));
+    if (!ws || ws_bytes < fb + fp32_part_bytes(g)) return ACH_EWORKSPACE;
     float *part = (float *)((char *)ws + fb);
     // a fully connected geometry reads the filter in its own layout, and so
     // does the patch-staged shallow-im2col kernel
@@ -3222,16 +3223,25 @@ size_t ach_conv_bwd_data_workspace(const ach_conv_desc *d)
     return (size_t)g.C * g.KS * g.KS * g.OH * g.OW * sizeof(float);
 }
 
+// bytes that ach_conv_bwd_data needs (the query adds what it makes use of)
+static size_t bwd_data_need(const ConvGeom &g, bool xy)
+{
+    if (xy) return xy_col_bytes(g);
+    if (g.S == 1 && g.P <= g.KS - 1)
+        return align256((size_t)g.F * g.C * g.KS * g.KS * sizeof(float)) +
+               fp32_part_bytes(dgrad_as_fwd(g), false);
+    return (size_t)g.C * g.KS * g.KS * g.OH * g.OW * sizeof(float);
+}
+
 int ach_conv_bwd_data(const ach_conv_desc *d, const float *dy, const float *w, float *dx,
                       void *ws, size_t ws_bytes, ach_stream_t stream)
 {
     if (!conv_ok(d) || !dy || !w || !dx) return ACH_EINVAL;
     if (!fits_int(d)) return ACH_EUNSUPPORTED;
-    const size_t need = ach_conv_bwd_data_workspace(d);
-    if (!ws || ws_bytes < need) return ACH_EWORKSPACE;
     const ConvGeom g = geom(d);
     hipStream_t st = as_stream(stream);
     const bool xy = conv_xy(d);
+    if (!ws || ws_bytes < bwd_data_need(g, xy)) return ACH_EWORKSPACE;
     if (!xy && dgrad_small_c(g) && !fc_geom(g)) return dgrad_small_c_launch(g, dy, w, dx, st);
     if (!xy && g.S == 1 && g.P <= g.KS - 1) {
         const size_t tot = (size_t)g.F * g.C * g.KS * g.KS;
@@ -3381,11 +3391,9 @@ int ach_conv_bwd_data_prepared(const ach_conv_desc *d, const float *dy, const fl
                     Epi(), false, false);
 }
 
-size_t ach_conv_bwd_filter_workspace(const ach_conv_desc *d)
+// bytes that the fp32 weight gradient needs
+static size_t fp32_wgrad_bytes(const ConvGeom &g)
 {
-    if (!conv_ok(d)) return 0;
-    const ConvGeom g = geom(d);
-    if (conv_xy(d)) return xy_col_bytes(g);
     // (the one-pass 1x1 kernel needs none, but unaligned operands take the
     // GEMM, so its workspace is reported)
     int splits, kchunk;
@@ -3393,6 +3401,18 @@ size_t ach_conv_bwd_filter_workspace(const ach_conv_desc *d)
     if (splits <= 1) return 0;
     const int groups = splits > 2 * SPLIT_GROUP ? (splits + SPLIT_GROUP - 1) / SPLIT_GROUP : 0;
     return (size_t)(splits + groups) * g.F * g.C * g.KS * g.KS * sizeof(float);
+}
+
+size_t ach_conv_bwd_filter_workspace(const ach_conv_desc *d)
+{
+    if (!conv_ok(d)) return 0;
+    const ConvGeom g = geom(d);
+    if (conv_xy(d)) return xy_col_bytes(g);
+    const size_t need = fp32_wgrad_bytes(g);
+    const WsplitPlan wp = wsplit_plan(g, 1 << 30);
+    if (!wp.ok) return need;
+    const size_t n = (size_t)wp.splits * g.F * g.C * g.KS * g.KS * sizeof(float);
+    return n > need ? n : need;
 }
 
 // dw += the weight gradient; with sgd.w, then the weights' SGD step on
@@ -3417,12 +3437,19 @@ static int bwd_filter(const ach_conv_desc *d, const float *x, const float *dy, f
     const int bm = wgrad_bm(g), bn = wgrad_bn(g);
     int splits, kchunk;
     wgrad_split(g, bm, bn, splits, kchunk);
-    const size_t need = ach_conv_bwd_filter_workspace(d);
+    const size_t need = fp32_wgrad_bytes(g);
     if (need && (!ws || ws_bytes < need)) return ACH_EWORKSPACE;
     hipStream_t st = as_stream(stream);
     float *part = (float *)ws;
     int rc;
     bool done = false;  // the update was applied in the GEMM's epilogue
+    // the three-piece kernel, with the slices that the workspace holds
+    const size_t held = ws ? ws_bytes / ((size_t)g.F * g.C * g.KS * g.KS * sizeof(float)) : 0;
+    const WsplitPlan wp = wsplit_plan(g, held > 1 << 20 ? 1 << 20 : (int)held);
+    if (wp.ok) {
+        rc = wsplit_launch(g, wp, x, dy, part, st);
+        return rc ? rc : wsplit_reduce(g, wp, part, dw, sgd, st);
+    }
     if (fc_geom(g)) rc = fc_wgrad_launch(g, x, dy, dw, part, bm, splits, kchunk, st, sgd, done);
     else if (bn == 32) rc = wgrad_launch<128, 32>(g, x, dy, dw, part, splits, kchunk, st, sgd, done);
     else if (bn == 64) rc = wgrad_launch<128, 64>(g, x, dy, dw, part, splits, kchunk, st, sgd, done);

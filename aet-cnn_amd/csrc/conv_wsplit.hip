@@ -1,0 +1,454 @@
+// Weight gradient of stride-1 convolutions that keep their size (k odd,
+// pad (k-1)/2): dW[f][c][ki][kj] = sum over images and positions of
+// dy[f][oy][ox] * x[c][oy+ki-P][ox+kj-P], on the bf16 matrix cores with
+// three exact bf16 pieces per float (the arithmetic of conv_split.hip).
+//
+// The contraction runs over positions, which are contiguous in both tensors,
+// so an operand fragment (8 consecutive positions of one row of f or c) is a
+// 16-byte LDS read and a tap's kj is a shift of x by whole elements.  A K
+// step is one input row y of a unit: 16 positions as two segments of 8,
+// either adjacent columns of one image or, when the row has an odd number of
+// segments, the same segment of two images.  At a step a wave reads x's row
+// once, forms its k shifted versions in registers (a segment keeps its two
+// neighbours on each side beside it) and multiplies them with the dy rows
+// y-ki+P of a ring in LDS: one x row and one dy row are split and staged per
+// step for k*k taps of MFMAs.  Rows of consecutive units follow each other
+// in the ring, so a slice is any range of steps.
+//
+// A workgroup is 64 filters x 64 channels x 9 taps: two groups of four waves
+// take halves of a slice's steps, each wave 32 x 32 x 9 (144 accumulator
+// registers), and add their sums in LDS, which halves the partial sums
+// written per CU.  A step's staging is spread over all lanes (each one
+// segment of one row, loaded a step ahead, split beside the MFMAs); dy rows
+// outside the image are read from a row of zeros, so a step has no branch.
+//
+// Bound: the matrix pipe beside the staging; 2.4 us per step of 54 MFMAs on
+// each of two waves per SIMD (1.44 us at the full clock).  Measured with the
+// reduction, batch 128, fp32 kernel before -> now: 128 -> 128 @ 32x32 293 ->
+// 189 us (205 TFLOP/s), 512 -> 512 @ 8x8 295 -> 187, 384 -> 384 @ 13x13 477
+// -> 325 (rows of 13 of 16 positions); batch 32, 512 -> 512 @ 8x8 88 -> 69.
+// Partial sums laid out [tap][f][c], 32 channels a line: stored as dw is
+// ([f][c][tap], 36 bytes between lanes) the first of these took 237 us.
+#include "conv_wsplit.hpp"
+#include "pieces.hpp"
+
+namespace ach {
+
+struct Wsplit {
+    const float *x, *dy;
+    float *part;
+    int B, C, H, W, F;
+    int S;         // steps: units * H
+    int spw;       // steps per group
+    int pair;      // the two segments are of two images
+    int nu;        // units per image (pair)
+    int cols;      // columns per unit
+    int mt, ct, tiles;
+    FastDiv dh, dnu;
+};
+
+// W8: rows of a multiple of 8 positions (whole segments, 16-byte loads)
+template <bool W8>
+__global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
+{
+    constexpr int KS = 3, P = 1, NT = 256, T = KS * KS;
+    constexpr int R = 64;                      // rows of dy (f) and of x (c) per workgroup
+    constexpr int ROWB = 6 * R * 16;           // bytes of a staged row: [piece][seg][r] x 16
+    constexpr int NBB = 12 * R * 4;            // its neighbour pairs: [piece][seg][side][r] x 4
+    constexpr int NR = KS + 1;                 // dy rows in the ring
+    constexpr int GB = (NR + 1) * ROWB + 2 * (ROWB + NBB) + NBB;
+    extern __shared__ __align__(16) char smem[];
+    const int grp = __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
+    const int tid = (int)threadIdx.x - grp * NT;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wf = wave & 1, wc = wave >> 1;
+    const int half = lane >> 5, l32 = lane & 31;
+    // a group's stages: the dy ring, a row of zeros, two x rows with their
+    // neighbours, a spare neighbour block
+    char *const dyb = smem + grp * GB, *const zero = dyb + NR * ROWB;
+    char *const xb = zero + ROWB;
+
+    // XCD x runs a contiguous range of (slice, tile) pairs, tiles fastest: the
+    // tiles of a slice share its rows of x and dy in that XCD's L2
+    int id = blockIdx.x + blockIdx.y * gridDim.x;
+    {
+        const int G = gridDim.x * gridDim.y, g8 = G >> 3, r8 = G & 7, xcd = id & 7, k = id >> 3;
+        id = xcd * g8 + min(xcd, r8) + k;
+    }
+    const int z = id / p.tiles;
+    id -= z * p.tiles;
+    const int c0 = (id % p.ct) * R, m0 = (id / p.ct) * R;
+    const int s0 = min(p.S, (z * 2 + grp) * p.spw), s1 = min(p.S, s0 + p.spw);
+    const int HW = p.H * p.W;
+
+    // Staging: waves 0 and 1 take 32 rows of dy each, 2 and 3 of x; a lane one
+    // segment (8 positions) of one row, and for x the two positions on each
+    // side of it.  A wave's role is a matter of operands, not of branches.
+    const bool isx = wave >= 2;
+    const int trow = (wave & 1) * 32 + (lane >> 1), seg = lane & 1;
+    const int nrow = isx ? p.C : p.F, row = (isx ? c0 : m0) + trow;
+    const __amdgpu_buffer_rsrc_t rs =
+        make_rsrc(isx ? p.x : p.dy, (unsigned)((size_t)p.B * nrow * HW * 4));
+    // (readfirstlane hides the role from the optimiser, which would turn the
+    // loop body into a branch per role)
+    auto role = [&](int x, int d) { return __builtin_amdgcn_readfirstlane(isx ? x : d); };
+    const int lead = role(0, P);  // step s brings x row s and dy row s + P
+    const int slot0 = role((NR + 1) * ROWB, 0), slotm = role(1, NR - 1);
+    const int slotb = role(ROWB + NBB, ROWB), slotn = role(0, P + NR);
+    const int nb0 = role((NR + 2) * ROWB, (NR + 3) * ROWB + 2 * NBB), nbb = role(ROWB + NBB, 0);
+    const int side = role(0, (int)kOOB);
+    const int ps = p.pair ? 1 : 0, segc = ps ? 0 : seg * 8, segb = ps ? seg : 0;
+    const int lanebase = (row + segb * nrow) * HW + segc;
+    char *const st0 = dyb + (trow + seg * R) * 16;
+    char *const st1 = dyb + (seg * 2 * R + trow) * 4;
+    auto load = [&](int s, float *r) {
+        const int ds = s + lead, dc = max(ds, 0);
+        const int u = fdiv(dc, p.dh), y = dc - u * p.H, q = fdiv(u, p.dnu);
+        const int cu = (u - q * p.nu) * p.cols, b0 = q << ps;
+        const int rows = (unsigned)ds < (unsigned)p.S ? nrow : 0;
+        const int col = cu + segc, left = p.W - col;
+        const bool ok = (row < rows) & (b0 + segb < p.B);
+        const int base = (lanebase + b0 * nrow * HW + y * p.W + cu) * 4;
+        if constexpr (W8) {
+            const int o = (ok & (left > 0)) ? base : (int)kOOB;
+            const float4 a = bload4_so(rs, o, 0), b = bload4_so(rs, o, 16);
+            r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w;
+            r[4] = b.x; r[5] = b.y; r[6] = b.z; r[7] = b.w;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) r[j] = bload(rs, (ok & (left > j)) ? base + 4 * j : (int)kOOB);
+        }
+        // the neighbours (a dy row has none: out-of-range offsets)
+        r[8] = bload(rs, ((ok & (col > 0) & (left > -2)) ? base - 8 : (int)kOOB) | side);
+        r[9] = bload(rs, ((ok & (col > 0) & (left > -1)) ? base - 4 : (int)kOOB) | side);
+        r[10] = bload(rs, ((ok & (left > 8)) ? base + 32 : (int)kOOB) | side);
+        r[11] = bload(rs, ((ok & (left > 9)) ? base + 36 : (int)kOOB) | side);
+    };
+    auto store = [&](int s, const float *r) {
+        v4u pc[3];
+        split8(r, pc);
+        const int slot = (s + slotn) & slotm;
+        char *const dst = st0 + slot0 + slot * slotb;
+        unsigned *const nb = reinterpret_cast<unsigned *>(st1 + nb0 + slot * nbb);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *reinterpret_cast<v4u *>(dst + q * 2 * R * 16) = pc[q];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float a = r[8 + 2 * i], b = r[9 + 2 * i];
+            const unsigned h = pk_bf16(a, b);
+            const float ra = a - bf_lo(h), rb = b - bf_hi(h);
+            const unsigned m = pk_bf16(ra, rb);
+            nb[i * R] = h;
+            nb[4 * R + i * R] = m;
+            nb[8 * R + i * R] = pk_bf16(ra - bf_lo(m), rb - bf_hi(m));
+        }
+    };
+
+    v16f acc[KS][KS];
+#pragma unroll
+    for (int i = 0; i < KS; ++i)
+#pragma unroll
+        for (int j = 0; j < KS; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+    for (int i = tid * 16; i < ROWB; i += NT * 16) *reinterpret_cast<v4u *>(zero + i) = v4u{0, 0, 0, 0};
+    // steps s0-2 and s0-1 bring the ring's first dy rows (their x rows go to
+    // slots that later steps overwrite)
+    float r[12];
+    {
+        float r0[12], r1[12], r2[12];
+        load(s0 - 2, r0);
+        load(s0 - 1, r1);
+        load(s0, r2);
+        load(s0 + 1, r);
+        store(s0 - 2, r0);
+        store(s0 - 1, r1);
+        store(s0, r2);
+    }
+    __syncthreads();
+    // every group runs p.spw iterations, one past its last step on rows that
+    // read as zero
+    int y = s0 - fdiv(s0, p.dh) * p.H;
+    const unsigned frag = (half * R + l32) * 16;
+    for (int s = s0; s < s0 + p.spw; ++s) {
+        const char *const xr = xb + (s & 1) * (ROWB + NBB);
+        v4u u[3], a[2][3];
+        unsigned nl[3], nr[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            u[q] = *reinterpret_cast<const v4u *>(xr + frag + (q * 2 * R + wc * 32) * 16);
+            const unsigned *nb = reinterpret_cast<const unsigned *>(xr + ROWB) +
+                                 (q * 2 + half) * 2 * R + wc * 32 + l32;
+            nl[q] = nb[0];
+            nr[q] = nb[R];
+        }
+        // tap ki reads dy row y - ki + P, or zeros beyond the image (and past
+        // the slice's end)
+        const unsigned live = s < s1 ? (unsigned)p.H : 0u;
+        auto load_a = [&](int i) {
+            const int slot = ((s - i + P + NR) & (NR - 1)) * ROWB;
+            const int in = -(int)((unsigned)(y - i + P) < live);  // all ones or zero
+            const char *const dr = dyb + ((slot & in) | (NR * ROWB & ~in));
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                a[i & 1][q] = *reinterpret_cast<const v4u *>(dr + frag + (q * 2 * R + wf * 32) * 16);
+        };
+        load_a(0);
+        v4u b[KS][3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const v4u v = u[q];
+            const unsigned m0_ = __builtin_amdgcn_alignbit(v[1], v[0], 16);
+            const unsigned m1_ = __builtin_amdgcn_alignbit(v[2], v[1], 16);
+            const unsigned m2_ = __builtin_amdgcn_alignbit(v[3], v[2], 16);
+            b[0][q] = v4u{__builtin_amdgcn_alignbit(v[0], nl[q], 16), m0_, m1_, m2_};
+            b[1][q] = v;
+            b[2][q] = v4u{m0_, m1_, m2_, __builtin_amdgcn_alignbit(nr[q], v[3], 16)};
+        }
+        // the rows of step s + 1, loaded a step ago, are split and stored and
+        // those of step s + 2 loaded beside the MFMAs
+        store(s + 1, r);
+        load(s + 2, r);
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            if (i + 1 < KS) load_a(i + 1);
+            const v4u *ca = a[i & 1];
+            // by product over all taps: no MFMA waits for the one before it
+#define ACH_TAPS(qa, qb)                                                                  \
+    _Pragma("unroll") for (int j = 0; j < KS; ++j)                                        \
+        acc[i][j] = MFMA_BF(as_bf(ca[qa]), as_bf(b[j][qb]), acc[i][j]);
+            ACH_TAPS(2, 0) ACH_TAPS(0, 2) ACH_TAPS(1, 1) ACH_TAPS(1, 0) ACH_TAPS(0, 1)
+            ACH_TAPS(0, 0)
+#undef ACH_TAPS
+        }
+#pragma unroll
+        for (int i = 0; i < 6 * T; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        }
+        if (++y == p.H) y = 0;
+        __syncthreads();
+    }
+
+    bool bad = false;
+#pragma unroll
+    for (int q = 0; q < T; ++q)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) bad |= !(fabsf(acc[q / KS][q % KS][e]) <= 3.402823466e38f);
+    const int c = c0 + wc * 32 + l32, f = m0 + wf * 32 + 4 * half;
+    if (__ballot(bad)) {  // rare: recompute this wave's tiles in fp32
+#pragma unroll
+        for (int q = 0; q < T; ++q) {
+            v16f a;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) a[e] = 0.f;
+#pragma unroll 1
+            for (int s = s0; s < s1; ++s) {
+                const int un = fdiv(s, p.dh), iy = s - un * p.H, im = fdiv(un, p.dnu);
+                const int oy = iy - q / KS + P, cb = (un - im * p.nu) * p.cols;
+                if (oy < 0 || oy >= p.H) continue;
+#pragma unroll 1
+                for (int e = 0; e < 16; ++e) {
+                    const int b = p.pair ? 2 * im + (e >> 3) : im;
+                    const int ox = cb + (p.pair ? e & 7 : e), ix = ox + q % KS - P;
+                    if (b >= p.B || ox >= p.W) continue;
+                    float xv = 0.f;
+                    if (c < p.C && ix >= 0 && ix < p.W)
+                        xv = p.x[(((size_t)b * p.C + c) * p.H + iy) * p.W + ix];
+#pragma unroll
+                    for (int g = 0; g < 16; ++g) {
+                        const int fr = f + 8 * (g >> 2) + (g & 3);
+                        if (fr < p.F)
+                            a[g] += p.dy[(((size_t)b * p.F + fr) * p.H + oy) * p.W + ox] * xv;
+                    }
+                }
+            }
+            acc[q / KS][q % KS] = a;
+        }
+    }
+    // the groups exchange tiles in rounds of QR taps: group q & 1 stores tap q
+    constexpr int QR = 4;
+    float4 *const xs = reinterpret_cast<float4 *>(smem);
+#pragma unroll
+    for (int q0 = 0; q0 < T; q0 += QR) {
+        if (q0) __syncthreads();
+#pragma unroll
+        for (int q = q0; q < (q0 + QR < T ? q0 + QR : T); ++q)
+            if ((q & 1) != grp) {
+                const v16f &t = acc[q / KS][q % KS];
+#pragma unroll
+                for (int r4 = 0; r4 < 4; ++r4)
+                    xs[((q - q0) * 4 + r4) * NT + tid] =
+                        make_float4(t[4 * r4], t[4 * r4 + 1], t[4 * r4 + 2], t[4 * r4 + 3]);
+            }
+        __syncthreads();
+#pragma unroll
+        for (int q = q0; q < (q0 + QR < T ? q0 + QR : T); ++q)
+            if ((q & 1) == grp) {
+                const v16f &t = acc[q / KS][q % KS];
+                const int ld = p.C;
+                float *base = p.part + (((size_t)z * T + q) * p.F + f) * ld + c;
+#pragma unroll
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    const float4 o = xs[((q - q0) * 4 + r4) * NT + tid];
+                    const float v[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (c < p.C && f + 8 * r4 + e < p.F)
+                            base[(size_t)(8 * r4 + e) * ld] = t[4 * r4 + e] + v[e];
+                }
+            }
+    }
+}
+
+// dw[f][c][t] += sum over z of part[z][t][f][c], z ascending within quarters
+// of the slices and the quarters' sums in order, then the SGD step when sg.w.
+// A block takes 64 channels of one filter: its four waves sum a quarter of
+// the slices each (64 consecutive channels per load), and the 64 x 9 results
+// are consecutive in dw.
+__global__ void __launch_bounds__(256) k_wsplit_reduce(const float *__restrict__ part,
+                                                       float *__restrict__ dw, int F, int C,
+                                                       int splits, Sgd sg)
+{
+    constexpr int T = 9;
+    __shared__ float sums[4][64][T];
+    const int f = blockIdx.y, c0 = blockIdx.x * 64;
+    const int lane = threadIdx.x & 63, zq = threadIdx.x >> 6, c = c0 + lane;
+    const int zs = (splits + 3) / 4, z0 = min(splits, zq * zs), z1 = min(splits, z0 + zs);
+    if (c < C) {
+        const size_t zstep = (size_t)T * F * C, tstep = (size_t)F * C;
+        const float *p = part + (size_t)f * C + c;
+        float s[T];
+#pragma unroll
+        for (int t = 0; t < T; ++t) s[t] = 0.f;
+        int z = z0;
+        for (; z + 2 <= z1; z += 2) {
+            float v[2][T];
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int t = 0; t < T; ++t) v[u][t] = p[(z + u) * zstep + t * tstep];
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int t = 0; t < T; ++t) s[t] += v[u][t];
+        }
+        if (z < z1) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) s[t] += p[z * zstep + t * tstep];
+        }
+#pragma unroll
+        for (int t = 0; t < T; ++t) sums[zq][lane][t] = s[t];
+    }
+    __syncthreads();
+    const int n = min(64, C - c0) * T;
+    float *d = dw + ((size_t)f * C + c0) * T;
+    float *w = sg.w ? sg.w + ((size_t)f * C + c0) * T : nullptr;
+    const float *q = &sums[0][0][0];
+    for (int i = threadIdx.x; i < n; i += 256) {
+        float o = d[i] + (((q[i] + q[64 * T + i]) + q[128 * T + i]) + q[192 * T + i]);
+        if (w) {
+            float a = w[i];
+            sgd_step(a, o, sg.dc, sg.lc, sg.mom);
+            w[i] = a;
+        }
+        d[i] = o;
+    }
+}
+
+int wsplit_reduce(const ConvGeom &g, const WsplitPlan &pl, const float *part, float *dw,
+                  const Sgd &sg, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_wsplit_reduce, dim3((g.C + 63) / 64, g.F), dim3(256), 0, st, part, dw, g.F,
+                       g.C, pl.splits, sg);
+    return check_launch();
+}
+
+static int wsplit_go(Wsplit &p, const WsplitPlan &pl, hipStream_t st)
+{
+    constexpr int R = 64, ROWB = 6 * R * 16, NBB = 12 * R * 4;
+    p.mt = (p.F + R - 1) / R;
+    p.ct = (p.C + R - 1) / R;
+    p.tiles = p.mt * p.ct;
+    const size_t lds = 2 * (size_t)(5 * ROWB + 2 * (ROWB + NBB) + NBB);
+    auto kern = p.W % 8 == 0 ? &k_conv_wsplit<true> : &k_conv_wsplit<false>;
+    const int rc = check(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    if (rc) return rc;
+    hipLaunchKernelGGL(kern, dim3(p.tiles, pl.splits), dim3(512), lds, st, p);
+    return check_launch();
+}
+
+// units per image (pair), columns per unit and whether segments pair images
+static void wsplit_units(const ConvGeom &g, int &pair, int &nu, int &cols, long long &units)
+{
+    const int segs = (g.W + 7) / 8;
+    pair = (segs & 1) && g.B > 1;
+    nu = pair ? segs : (segs + 1) / 2;
+    cols = pair ? 8 : 16;
+    units = (long long)(pair ? (g.B + 1) / 2 : g.B) * nu;
+}
+
+WsplitPlan wsplit_plan(const ConvGeom &g, int room)
+{
+    WsplitPlan pl{};
+    if (g.S != 1 || g.KS != 3 || 2 * g.P != g.KS - 1 || g.OH != g.H || g.OW != g.W) return pl;
+    int pair, nu, cols;
+    long long units;
+    wsplit_units(g, pair, nu, cols, units);
+    const long long S = units * g.H;
+    if (S >= (1ll << 26)) return pl;
+    const long long tiles = (long long)((g.F + 63) / 64) * ((g.C + 63) / 64);
+    // Time model (us), fitted to a sweep of layer shapes: a step of the two
+    // groups' eight waves; more where the rows are not whole segments, and
+    // where a line of memory holds several units' segments of an image pair,
+    // which are read far apart (the line comes from HBM for each); the
+    // partial sums written and read; and prologue, exchange and reduction.
+    // The fp32 kernel: 125 TFLOP/s and 9 us.
+    const double step = pair && nu >= 3 ? (nu >= 5 ? 4.4 : 3.5) : (g.W % 8 ? 2.7 : 2.4);
+    const double mn4 = (double)g.F * g.C * g.KS * g.KS * 4;
+    const double fp32 = 9.0 + 2e-6 / 125 * g.B * g.H * g.W * (mn4 / 4);
+    if (0.95 * fp32 < 12.0 + 4 * step + 4.0) return pl;  // the shortest plan is no faster
+    double best = -1;
+    for (int k = 1; k <= 10; ++k) {  // one to six rounds of 256 workgroups, or a part of one
+        const int s = k <= 6 ? (int)(256 * k / tiles) : (int)(256 / ((k - 5) * tiles));
+        if (s < 1 || s > room) continue;
+        const long long spw = (S + 2 * s - 1) / (2 * s);
+        if (s > 1 && spw < 4) continue;
+        const long long rounds = (tiles * s + 255) / 256;
+        const double t = 12.0 + rounds * (spw * step + 4.0) + s * mn4 * 2 / 5e6;
+        if (best < 0 || t < best * 0.995) {
+            best = t;
+            pl.splits = s;
+            pl.spw = (int)spw;
+        }
+    }
+    if (best < 0 && room >= 1) {  // more tiles than workgroups to fill the chip
+        pl.splits = 1;
+        pl.spw = (int)((S + 1) / 2);
+        best = 12.0 + (tiles + 255) / 256 * (pl.spw * step + 4.0) + mn4 * 2 / 5e6;
+    }
+    pl.ok = best >= 0 && best < 0.95 * fp32;
+    return pl;
+}
+
+int wsplit_launch(const ConvGeom &g, const WsplitPlan &pl, const float *x, const float *dy,
+                  float *part, hipStream_t st)
+{
+    Wsplit p{};
+    p.x = x; p.dy = dy; p.part = part;
+    p.B = g.B; p.C = g.C; p.H = g.H; p.W = g.W; p.F = g.F;
+    long long units;
+    wsplit_units(g, p.pair, p.nu, p.cols, units);
+    p.S = (int)(units * g.H);
+    p.spw = pl.spw;
+    p.dh = make_fastdiv((unsigned)g.H);
+    p.dnu = make_fastdiv((unsigned)p.nu);
+    return wsplit_go(p, pl, st);
+}
+
+}  // namespace ach

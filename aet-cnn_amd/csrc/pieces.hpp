@@ -1,0 +1,42 @@
+// Exact three-piece bf16 operands (see conv_split.hip for the arithmetic).
+#pragma once
+
+#include "conv_common.hpp"
+
+namespace ach {
+
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
+// bf16 pair (lo = a, hi = b), rounded to nearest even
+__device__ __forceinline__ unsigned pk_bf16(float a, float b)
+{
+    const v2f v = {a, b};
+    const v2bf r = __builtin_convertvector(v, v2bf);
+    return __builtin_bit_cast(unsigned, r);
+}
+__device__ __forceinline__ float bf_lo(unsigned u) { return __uint_as_float(u << 16); }
+__device__ __forceinline__ float bf_hi(unsigned u) { return __uint_as_float(u & 0xffff0000u); }
+
+// eight floats -> three pieces of eight bf16 (f = p[0] + p[1] + p[2] exactly)
+__device__ __forceinline__ void split8(const float *f, v4u *p)
+{
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = f[2 * i], b = f[2 * i + 1];
+        const unsigned h = pk_bf16(a, b);
+        const float ra = a - bf_lo(h), rb = b - bf_hi(h);
+        const unsigned m = pk_bf16(ra, rb);
+        p[0][i] = h;
+        p[1][i] = m;
+        p[2][i] = pk_bf16(ra - bf_lo(m), rb - bf_hi(m));
+    }
+}
+
+__device__ __forceinline__ v8bf as_bf(v4u v) { return __builtin_bit_cast(v8bf, v); }
+
+#define MFMA_BF(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0)
+
+}  // namespace ach

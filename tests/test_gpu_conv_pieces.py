@@ -1,6 +1,7 @@
 """The convolution kernels that take every float as three bf16 pieces
-(conv_split.hip): forward and input gradient against 64-bit references where
-their tiles, channel chunks and K parts end, and infinities and NaNs.
+(conv_split.hip, conv_wsplit.hip): forward, input gradient and weight
+gradient against 64-bit references where their tiles, channel chunks and K
+parts end, and infinities and NaNs.
 
 Bound, per output: the six piece products kept of a*b leave out less than
 2^-24 |ab|, and a matrix instruction adds 16 products with one rounding, so
@@ -94,3 +95,70 @@ def test_non_finite_and_largest_values(gpu, shape, value):
     near = fin & (abs(b) < 1e30)  # sums without the large value
     assert np.all(abs(a[near] - b[near]) <= 1e-5 * abs(b[near]).max())
     assert np.all(abs(a[fin] - b[fin]) <= 1e-5 * abs(b[fin]) + 1e-5 * abs(b[near]).max())
+
+
+# shapes large enough for the three-piece weight gradient
+WGRAD = [
+    (32, 512, 8, 8, 512),     # one segment per row: image pairs
+    (65, 256, 8, 8, 500),     # a last image without a partner, ragged filters
+    (64, 250, 13, 13, 384),   # rows of 13 of 16 positions, ragged channels
+    (1, 256, 128, 64, 256),   # one image, four units per row
+    (128, 64, 32, 32, 64),    # one tile, most slices
+]
+
+
+def wgrad_ref(x, dy):
+    B, Cc, H, W = x.shape
+    xp = np.pad(x, ((0, 0), (0, 0), (1, 1), (1, 1)))
+    out = np.zeros((dy.shape[1], Cc, 3, 3), x.dtype)
+    for i in range(3):
+        for j in range(3):
+            out[:, :, i, j] = np.tensordot(dy, xp[:, :, i:i + H, j:j + W],
+                                           axes=([0, 2, 3], [0, 2, 3]))
+    return out
+
+
+def run_wgrad(gpu, x, dy, dw0):
+    B, Cc, H, W = x.shape
+    d = aetcnn.ConvDesc(B, Cc, H, W, dy.shape[1], 3, 1, 1)
+    nb = gpu.ach_conv_bwd_filter_workspace(C.byref(d))
+    ws, dx, ddy, ddw = D(nb // 4 + 64), D.from_numpy(x), D.from_numpy(dy), D.from_numpy(dw0)
+    check(gpu.ach_conv_bwd_filter(C.byref(d), dx.ptr, ddy.ptr, ddw.ptr, ws.ptr, nb, None))
+    return ddw.numpy()
+
+
+@pytest.mark.parametrize("shape", WGRAD, ids=lambda s: "x".join(map(str, s)))
+def test_weight_gradient(gpu, shape):
+    """n = 6 roundings per 16 positions, random: 8 standard deviations of
+    sqrt(n) half-ulps of the largest partial sum."""
+    B, Cc, H, W, F = shape
+    rng = np.random.default_rng(sum(shape))
+    x = rng.standard_normal((B, Cc, H, W)).astype(np.float32)
+    dy = rng.standard_normal((B, F, H, W)).astype(np.float32)
+    dw0 = rng.standard_normal((F, Cc, 3, 3)).astype(np.float32)
+    got = run_wgrad(gpu, x, dy, dw0).astype(np.float64)
+    x, dy = x.astype(np.float64), dy.astype(np.float64)
+    ref = dw0 + wgrad_ref(x, dy)
+    # the partial sums' size: the norms of the products' rows
+    size = np.sqrt(wgrad_ref(x * x, dy * dy)) + abs(dw0)
+    n = 6 * B * H * -(-W // 8) / 2 + 64
+    assert np.all(abs(got - ref) <= 8 * n ** 0.5 * 2.0 ** -25 * size)
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_weight_gradient_non_finite(gpu, value):
+    """One non-finite input reaches its channel's nine taps of every filter
+    and nothing else, as in fp32 arithmetic."""
+    B, Cc, H, W, F = WGRAD[0]
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((B, Cc, H, W)).astype(np.float32)
+    dy = rng.standard_normal((B, F, H, W)).astype(np.float32)
+    x[5, 70, 3, 3] = value
+    got = run_wgrad(gpu, x, dy, np.zeros((F, Cc, 3, 3), np.float32))
+    want = np.zeros(got.shape, bool)
+    want[:, 70] = True
+    assert np.array_equal(~np.isfinite(got), want)
+    if np.isinf(value):  # its sign: that of the dy it meets
+        for i in range(3):
+            for j in range(3):
+                assert np.array_equal(np.sign(got[:, 70, i, j]), np.sign(dy[5, :, 4 - i, 4 - j]))
