@@ -155,14 +155,13 @@ __global__ void __launch_bounds__(64 * WM * WN * KG, 2) k_conv_split(SplitFwd p)
     // A: this lane's filter row, channels half*8 .. +7 of the chunk
     const int m = m0 + wm * 32 + l32;
     const unsigned aoff = m < p.M ? (unsigned)(half * 8 * T * p.M + m) * 4u : kOOB;
-    float ar[8];
-    auto load_a = [&](int ch, int tap) {
+    auto load_a = [&](int ch, int tap, float *r) {
         const unsigned d = (unsigned)(chan0(ch) * T + tap) * (unsigned)p.M * 4u;
         const __amdgpu_buffer_rsrc_t rw =
             make_rsrc(reinterpret_cast<const char *>(p.wt) + d, wbytes - d);
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-            ar[j] = bload_so(rw, aoff, (unsigned)(j * T) * (unsigned)p.M * 4u);
+            r[j] = bload_so(rw, aoff, (unsigned)(j * T) * (unsigned)p.M * 4u);
     };
 
     // B: this lane's output columns
@@ -184,18 +183,23 @@ __global__ void __launch_bounds__(64 * WM * WN * KG, 2) k_conv_split(SplitFwd p)
 
     // every group of the workgroup runs p.cps chunks (a group past its last
     // chunk only joins the barriers)
+    // The filter pipeline: in tap t the pieces of tap t multiply, the raw
+    // values of tap t+1 are split and those of tap t+1+AD are loaded (the
+    // fewer MFMAs a tap has, the more taps it takes to cover a load).
+    constexpr int AD = 4 / NF;
+    float ar[AD][8];
+    v4u a[2][3];
     if (ch0 < ch1) {
+        float first[8];
         load_px(ch0);
-        load_a(ch0, 0);
+        load_a(ch0, 0, first);
+#pragma unroll
+        for (int t = 1; t <= AD; ++t) load_a(ch0, t, ar[t % AD]);
         store_px(stage);
+        split8(first, a[0]);
     }
     __syncthreads();
     int cur = 0;
-    // Tap t multiplies a[t & 1] while the raw filter values of tap t+1 are
-    // split into the other one and those of tap t+2 are loaded; a fragment's
-    // B pieces are read one fragment ahead.
-    v4u a[2][3];
-    if (ch0 < ch1) split8(ar, a[0]);
     auto compute = [&](const char *buf, int ch, bool next) {
         v4u b[2][3];
         auto load_b = [&](int step) {  // step = tap * NF + f
@@ -204,15 +208,15 @@ __global__ void __launch_bounds__(64 * WM * WN * KG, 2) k_conv_split(SplitFwd p)
 #pragma unroll
             for (int q = 0; q < 3; ++q) b[step & 1][q] = *reinterpret_cast<const v4u *>(src + q * 32);
         };
-        load_a(ch, 1);
         load_b(0);
 #pragma unroll
         for (int tap = 0; tap < T; ++tap) {
             __builtin_amdgcn_sched_barrier(0);
             const v4u *ca = a[tap & 1];
-            split8(ar, a[(tap + 1) & 1]);
-            if (tap + 2 < T) load_a(ch, tap + 2);
-            else if (tap + 2 == T) load_a(next ? ch + 1 : ch, 0);
+            split8(ar[(tap + 1) % AD], a[(tap + 1) & 1]);
+            const int ahead = tap + 1 + AD;
+            if (ahead < T) load_a(ch, ahead, ar[ahead % AD]);
+            else load_a(next ? ch + 1 : ch, ahead - T, ar[ahead % AD]);
 #pragma unroll
             for (int f = 0; f < NF; ++f) {
                 const int step = tap * NF + f;
@@ -233,9 +237,21 @@ __global__ void __launch_bounds__(64 * WM * WN * KG, 2) k_conv_split(SplitFwd p)
                 if (i % 3 == 0) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
             }
         }
-        if (T & 1) {
+        // the next chunk's tap 0 and the raw values move to where it expects
+        // them (the taps of a chunk are an odd number)
+        static_assert(T % 2 == 1 && T % AD == 1 % AD && T > AD, "slots of the filter pipeline");
 #pragma unroll
-            for (int q = 0; q < 3; ++q) a[0][q] = a[1][q];
+        for (int q = 0; q < 3; ++q) a[0][q] = a[1][q];
+        if constexpr (AD > 1) {
+            float t[AD][8];
+#pragma unroll
+            for (int i = 0; i < AD; ++i)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) t[i][j] = ar[(T + i) % AD][j];
+#pragma unroll
+            for (int i = 0; i < AD; ++i)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) ar[i][j] = t[i][j];
         }
     };
     for (int it = 0; it < p.cps; ++it) {
@@ -376,42 +392,56 @@ SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, int fp32_splits, int 
     SplitFwdPlan pl{};
     pl.ok = false;
     if (g.S != 1 || !(g.KS == 3 || g.KS == 5) || g.P > g.KS - 1 || g.C < SP_CH) return pl;
+    // chunks that are mostly repeated channels (17-22, 33) lose to the fp32
+    // kernel (18 -> 16 @ 39x39, batch 5: 9.9 against 11.0 us)
+    if (g.C < 0.7 * SP_CH * ((g.C + SP_CH - 1) / SP_CH)) return pl;
     if ((long long)g.B * (g.OH + g.KS) >= (1ll << 30)) return pl;
     const int M = g.F, N = g.B * g.OH * g.OW;
-    pl.wm = M <= 32 ? 1 : (M <= 64 ? 2 : (M <= 96 ? 3 : 4));
-    pl.wn = pl.wm == 1 ? 4 : (pl.wm == 2 ? 2 : 1);
-    const int nt = 64 * pl.wm * pl.wn;
     long long npx, nreal;
     split_patch(g, npx, nreal);
-    const long long tpt = (2 * nreal + nt - 1) / nt;
-    if (tpt > 4 || npx * SP_PXB > 150 * 1024) return pl;
+    if (npx * SP_PXB > 150 * 1024) return pl;
     pl.npx = (int)npx;
-    pl.tpt = tpt < 2 ? 2 : (int)tpt;
-    const int tiles = ((M + 32 * pl.wm - 1) / (32 * pl.wm)) * ((N + SP_BN - 1) / SP_BN);
-    const int nchunk = (g.C + SP_CH - 1) / SP_CH;
-    // K parts: the modelled time (us) of the rounds of workgroups, two per CU
-    // (or one with two K groups), plus the split-K reduction.  Measured:
-    // 11 us per 16-channel chunk of a 3x3 filter with two 128 x 128
-    // workgroups on every CU (128 -> 128 @ 32x32, batch 128), 0.65 of it
-    // with one.  Small grids take no more slices than the fp32 plan.
-    const double chunk_us = 11.0 * g.KS * g.KS / 9.0 / pl.wn;
+    const int nchunk = (g.C + SP_CH - 1) / SP_CH, nt = (N + SP_BN - 1) / SP_BN;
+    const int wide = M <= 32 ? 1 : (M <= 64 ? 2 : (M <= 96 ? 3 : 4));
+    const long long big = (long long)((M + 127) / 128) * nt;  // 128 x 128 tiles
+    // Waves along M and K parts: the modelled time (us) of the rounds of
+    // workgroups, two per CU (or one with two K groups), plus the split-K
+    // reduction.  Measured: 11 us per 16-channel chunk of a 3x3 filter with
+    // two 128 x 128 workgroups on every CU (128 -> 128 @ 32x32, batch 128),
+    // 0.65 of it with one; tiles of half and a quarter of the fragments per
+    // wave take 6.2 and 3.6 (every wave loads the filter rows again), down to
+    // about 2.2 us for the loads' latency, and win where the grid is small
+    // (a 13-layer net's inference of one image: 227 -> 201 us).  Small grids take no more slices than the fp32 plan.
     double best = -1;
-    for (int kg = 1; kg <= (kg_ok && pl.wm == 4 && pl.tpt <= 3 ? 2 : 1); ++kg)
-        for (int s = 1; s * kg <= nchunk && s <= 32; ++s) {
-            const int cps = (nchunk + s * kg - 1) / (s * kg);
-            const int splits = (nchunk + cps * kg - 1) / (cps * kg);
-            if (splits > 1 && (splits > room || (splits > fp32_splits && tiles < 128))) continue;
-            const long long wgs = (long long)tiles * splits;
-            const long long full = wgs / (512 / kg), rest = wgs % (512 / kg);
-            double t = full * cps * chunk_us;
-            if (rest) t += cps * chunk_us * (rest > 256 || kg == 2 ? 1.0 : 0.65);
-            if (splits > 1) t += 5.0 + (2.0 * splits + 1) * M * (double)N * 4 / 5e6;
-            if (best < 0 || t < best * 0.97) {
-                best = t;
-                pl.kg = kg;
-                pl.splits = splits;
+    for (int wm = wide; wm >= 1; wm = wm == 4 ? 2 : wm - 1) {
+        const int wn = wm == 1 ? 4 : (wm == 2 ? 2 : 1), thr = 64 * wm * wn;
+        const long long tpt = (2 * nreal + thr - 1) / thr;
+        const long long tiles = (long long)((M + 32 * wm - 1) / (32 * wm)) * nt;
+        if (tpt > 4 || tiles > 0x7fffffffLL) continue;
+        const double per9 = wn == 1 ? 11.0 : (wn == 2 ? 6.2 : 3.6), taps = g.KS * g.KS / 9.0;
+        const double paired = per9 * taps, single = (per9 * 0.65 > 2.2 ? per9 * 0.65 : 2.2) * taps;
+        for (int kg = 1; kg <= (kg_ok && wm == 4 && tpt <= 3 ? 2 : 1); ++kg)
+            for (const int s : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 24, 32}) {
+                if (s * kg > nchunk || (s > 1 && tiles * s > 2048)) break;
+                const int cps = (nchunk + s * kg - 1) / (s * kg);
+                const int splits = (nchunk + cps * kg - 1) / (cps * kg);
+                if (splits > 1 && (splits > room || (splits > fp32_splits && big < 128))) continue;
+                const long long wgs = tiles * splits;
+                const long long full = wgs >> (kg == 2 ? 8 : 9), rest = wgs & (kg == 2 ? 255 : 511);
+                double t = full * cps * paired;
+                if (rest) t += cps * (rest > 256 || kg == 2 ? paired : single);
+                if (splits > 1) t += 5.0 + (2.0 * splits + 1) * M * (double)N * 4 / 5e6;
+                if (best < 0 || t < best * 0.97) {
+                    best = t;
+                    pl.wm = wm;
+                    pl.wn = wn;
+                    pl.kg = kg;
+                    pl.splits = splits;
+                    pl.tpt = tpt < 2 ? 2 : (int)tpt;
+                }
             }
-        }
+    }
+    if (best < 0) return pl;
     const int one = (pl.npx + 1) * SP_PXB;
     // two workgroups (or two K groups) share a CU's 160 KB
     pl.nbuf = 2 * one <= 80 * 1024 ? 2 : 1;
