@@ -162,3 +162,35 @@ def test_weight_gradient_non_finite(gpu, value):
         for i in range(3):
             for j in range(3):
                 assert np.array_equal(np.sign(got[:, 70, i, j]), np.sign(dy[5, :, 4 - i, 4 - j]))
+
+
+@pytest.mark.parametrize("shape", [
+    # (B, C, H, W, F, k, s, p): input gradients by phases
+    (3, 48, 9, 7, 20, 3, 2, 1),
+    (2, 33, 8, 11, 70, 5, 2, 2),     # ragged channels: dword filter loads
+    (2, 130, 6, 6, 16, 3, 2, 1),     # 128-row tiles, ragged
+    (2, 8, 7, 9, 12, 1, 2, 0),       # three phases without taps: zeros
+    (2, 8, 10, 10, 12, 2, 3, 0),     # a window narrower than the stride
+    (1, 12, 13, 13, 9, 5, 4, 3),
+    (2, 5, 23, 17, 6, 11, 4, 0),
+    (2, 16, 5, 5, 8, 3, 2, 2),       # padding 2
+    (2, 4, 2, 3, 8, 2, 2, 0),        # one or two pixels per phase
+    (2, 6, 7, 7, 10, 3, 5, 1),       # a stride above the phases' limit
+], ids=lambda s: "x".join(map(str, s)))
+def test_strided_input_gradient(gpu, shape):
+    """fp32 sums of at most F*k*k products: |error| <= F k k 2^-24 sum |a||b|."""
+    B, Cc, H, W, F, k, s, p = shape
+    rng = np.random.default_rng(sum(shape))
+    w = rng.standard_normal((F, Cc, k, k)).astype(np.float32)
+    oh, ow = (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+    dy = rng.standard_normal((B, F, oh, ow)).astype(np.float32)
+    d = aetcnn.ConvDesc(B, Cc, H, W, F, k, s, p)
+    nb = gpu.ach_conv_bwd_data_workspace(C.byref(d))
+    ref = refs64.dgrad_ref(dy, w, (B, Cc, H, W), s, p)
+    mag = refs64.dgrad_ref(abs(dy), abs(w), (B, Cc, H, W), s, p)
+    dw, ddy = D.from_numpy(w), D.from_numpy(dy)
+    # with the queried workspace, and with one image's columns only
+    for n in (nb, Cc * k * k * oh * ow * 4):
+        ws, dx = D(n // 4 + 64), D.from_numpy(np.full((B, Cc, H, W), 7.0, np.float32))
+        check(gpu.ach_conv_bwd_data(C.byref(d), ddy.ptr, dw.ptr, dx.ptr, ws.ptr, n, None))
+        assert np.all(abs(dx.numpy() - ref) <= F * k * k * 2.0 ** -24 * mag)
