@@ -29,6 +29,7 @@
 // delta slice) run on the same XCD and share its L2.
 #include "conv_split.hpp"
 #include "conv_wsplit.hpp"
+#include "fc_split.hpp"
 
 #include <type_traits>
 
@@ -1048,14 +1049,17 @@ struct DgradPhase {
     using AL = typename std::conditional<VECA, AWeightsT4<BM, BK>, AWeightsT<BM, BK>>::type;
     using BLd = BPhase;
     const float *dy, *wp;
-    float *dx;
+    float *dx;  // or, with parts > 1, partial sums [part][dx]
     ConvGeom g;
-    int M, K;
+    int M, K, parts;
     PhaseTable tab;
+    // grid slice z: part z % parts of phase z / parts
     __device__ __forceinline__ void krange(int z, int &kb, int &ke) const
     {
-        kb = tab.p[z].k0;
-        ke = kb + tab.p[z].nk;
+        const Phase &ph = tab.p[z / parts];
+        const int end = ph.k0 + ph.nk, len = ((ph.nk + parts - 1) / parts + BK - 1) / BK * BK;
+        kb = min(end, ph.k0 + z % parts * len);
+        ke = min(end, kb + len);
     }
     __device__ __forceinline__ void init_a(AL &a, int m0, int tid, int) const { a.init(wp, M, K, m0, tid); }
     __device__ __forceinline__ void init_b(BPhase &b, int n0, int tid, int kb) const
@@ -1066,12 +1070,12 @@ struct DgradPhase {
     }
     __device__ __forceinline__ void store_tile(int mb, int n, const v16f &acc, int z, bool) const
     {
-        const Phase &ph = tab.p[z];
+        const Phase &ph = tab.p[z / parts];
         if (n >= ph.n) return;
         const int b = fdiv(n, ph.dhw), p = n - b * ph.h * ph.w;
         const int r = fdiv(p, ph.dw), c = p - r * ph.w;
         const size_t hw = (size_t)g.H * g.W;
-        float *base = dx + ((size_t)b * M + mb) * hw + (size_t)(r * g.S + ph.a) * g.W + c * g.S + ph.b;
+        float *base = dx + ((size_t)(z % parts * g.B + b) * M + mb) * hw + (size_t)(r * g.S + ph.a) * g.W + c * g.S + ph.b;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int dm = 8 * (e >> 2) + (e & 3);
@@ -2818,8 +2822,9 @@ static size_t fwd_part_bytes(const ConvGeom &g, bool kg_ok = true)
     const FwdPlan pl = fwd_plan(g, kg_ok);
     const SplitFwdPlan sp = split_fwd_plan(g, kg_ok, pl.pslices(), 1 << 30);
     const size_t need = fp32_part_bytes(g, kg_ok);
-    if (!sp.ok || sp.splits <= 1) return need;
-    const size_t n = (size_t)sp.splits * g.F * g.B * g.OH * g.OW * sizeof(float);
+    const int slices = fc_geom(g) ? fc_split_slices(g.B, g.F, g.C, 1 << 30) : sp.ok ? sp.splits : 0;
+    if (slices <= 1) return need;
+    const size_t n = (size_t)slices * g.F * g.B * g.OH * g.OW * sizeof(float);
     return n > need ? n : need;
 }
 
@@ -2953,12 +2958,17 @@ static int fwd_impl(const ConvGeom &g, const float *x, const float *w, float *y,
     const size_t room = part ? part_bytes / ((size_t)g.F * g.B * g.OH * g.OW * sizeof(float)) : 0;
     SplitFwdPlan sp = split_fwd_plan(g, kg_ok, pl.pslices(), room > 1024 ? 1024 : (int)room);
     sp.ok = sp.ok && pieces;
-    const int ps = sp.ok ? sp.splits : pl.pslices();
+    const int fc = pieces && fc_geom(g)
+                       ? fc_split_slices(g.B, g.F, g.C, room > 1024 ? 1024 : (int)room) : 0;
+    const int ps = fc ? fc : sp.ok ? sp.splits : pl.pslices();
     const bool unsplit = ps == 1;  // no partial sums
     const bool gemm_epi = e.active() && unsplit;
     int rc;
-    if (sp.ok) {
-        rc = split_fwd_launch(g, sp, x, w, y, part, e, st);
+    if (sp.ok || fc) {
+        // a fully connected filter is [F][K], or for the input gradient the
+        // k-major [K][F]
+        rc = fc ? fc_split_launch({x, g.B, false}, {w, g.F, !w_nat}, g.C, fc, y, part, e, st)
+                : split_fwd_launch(g, sp, x, w, y, part, e, st);
         if (rc || unsplit) return rc;
     } else if (gemm_epi) {
         if (pl.bm == 32) rc = fwd_bm<32, true>(g, pl, x, w, y, part, e, w_nat, st);
@@ -2967,7 +2977,7 @@ static int fwd_impl(const ConvGeom &g, const float *x, const float *w, float *y,
         else rc = fwd_bm<128, true>(g, pl, x, w, y, part, e, w_nat, st);
         return rc;
     }
-    if (sp.ok) rc = ACH_OK;
+    if (sp.ok || fc) rc = ACH_OK;
     else if (pl.bm == 32) rc = fwd_bm<32, false>(g, pl, x, w, y, part, e, w_nat, st);
     else if (pl.bm == 96) rc = fwd_bm_padded<96, false>(g, pl, x, w, y, part, e, st);
     else if (pl.bm == 64) rc = fwd_bm<64, false>(g, pl, x, w, y, part, e, w_nat, st);
@@ -3283,9 +3293,13 @@ static int dgrad_small_c_launch(const ConvGeom &g, const float *dy, const float 
 
 // the phases of a strided input gradient; every phase has at least one pixel
 // for strides up to the input's size
+// (and images whose own GEMM, k*k*C x OH*OW, fills the chip keep the
+// per-image passes: 320 <- 416 channels, 5x5 at 40x40: 69 us an image, 71 by
+// phases)
 static bool dgrad_phases(const ConvGeom &g)
 {
-    return g.S > 1 && g.S <= PH_MAX_S && g.S <= g.H && g.S <= g.W && !fc_geom(g);
+    const long long own = ((long long)g.C * g.KS * g.KS + 127) / 128 * ((g.OH * g.OW + 127) / 128);
+    return own < 240 && g.S > 1 && g.S <= PH_MAX_S && g.S <= g.H && g.S <= g.W && !fc_geom(g);
 }
 static PhaseTable phase_table(const ConvGeom &g)
 {
@@ -3318,29 +3332,62 @@ static PhaseTable phase_table(const ConvGeom &g)
 }
 template <int BM>
 static int dgrad_phases_bm(const ConvGeom &g, const PhaseTable &t, const float *dy, const float *wp,
-                           float *dx, int K, hipStream_t st)
+                           float *dx, int K, int parts, hipStream_t st)
 {
     const int nmax = t.p[0].n;  // phase (0, 0) has the most pixels
     if (g.C % 4 == 0) {
-        DgradPhase<BM, true> p{dy, wp, dx, g, g.C, K, t};
-        return launch_gemm(p, g.C, nmax, t.n, st);
+        DgradPhase<BM, true> p{dy, wp, dx, g, g.C, K, parts, t};
+        return launch_gemm(p, g.C, nmax, t.n * parts, st);
     }
-    DgradPhase<BM, false> p{dy, wp, dx, g, g.C, K, t};
-    return launch_gemm(p, g.C, nmax, t.n, st);
+    DgradPhase<BM, false> p{dy, wp, dx, g, g.C, K, parts, t};
+    return launch_gemm(p, g.C, nmax, t.n * parts, st);
 }
-// wp: F*C*k*k floats of workspace
+// K parts of every phase: enough for two workgroups per CU, eight k-tiles each
+// on average (320 <- 416 channels, 5x5 stride 2 at 40x40, batch 3: 120
+// workgroups of 234 k-tiles took 385 us)
+static int dgrad_parts(const ConvGeom &g)
+{
+    const int bm = g.C <= 32 ? 32 : (g.C <= 64 ? 64 : 128), ph = g.S * g.S;
+    const long long n0 = (long long)g.B * ((g.H + g.S - 1) / g.S) * ((g.W + g.S - 1) / g.S);
+    const long long wgs = (g.C + bm - 1) / bm * ((n0 + 127) / 128) * ph;
+    const long long kt = (long long)g.F * g.KS * g.KS / ph / 16;
+    long long p = 512 / wgs;
+    if (p > kt / 8) p = kt / 8;
+    return p < 1 ? 1 : (p > 16 ? 16 : (int)p);
+}
+static size_t phase_filter_bytes(const ConvGeom &g)
+{
+    return ((size_t)g.F * g.C * g.KS * g.KS * sizeof(float) + 255) & ~(size_t)255;
+}
+// ws: the filter by phases, then the parts' sums where they fit
 static int dgrad_phases_launch(const ConvGeom &g, const float *dy, const float *w, float *dx,
-                               float *wp, hipStream_t st)
+                               void *ws, size_t ws_bytes, hipStream_t st)
 {
     const PhaseTable t = phase_table(g);
     const int K = g.F * g.KS * g.KS, total = K * g.C;
+    float *const wp = (float *)ws;
     hipLaunchKernelGGL(k_phase_filters, dim3((total + 255) / 256), dim3(256), 0, st, w, wp, g.C,
                        g.KS, g.S, total, make_fastdiv((unsigned)g.C), t);
-    const int rc = check_launch();
+    int rc = check_launch();
     if (rc) return rc;
-    if (g.C <= 32) return dgrad_phases_bm<32>(g, t, dy, wp, dx, K, st);
-    if (g.C <= 64) return dgrad_phases_bm<64>(g, t, dy, wp, dx, K, st);
-    return dgrad_phases_bm<128>(g, t, dy, wp, dx, K, st);
+    const size_t n = (size_t)g.B * g.C * g.H * g.W, fb = phase_filter_bytes(g);
+    int parts = dgrad_parts(g);
+    if (ws_bytes < fb + parts * n * sizeof(float)) parts = 1;
+    float *const part = (float *)((char *)ws + fb), *const out = parts > 1 ? part : dx;
+    if (g.C <= 32) rc = dgrad_phases_bm<32>(g, t, dy, wp, out, K, parts, st);
+    else if (g.C <= 64) rc = dgrad_phases_bm<64>(g, t, dy, wp, out, K, parts, st);
+    else rc = dgrad_phases_bm<128>(g, t, dy, wp, out, K, parts, st);
+    if (rc || parts == 1) return rc;
+    const bool v4 = (n & 3) == 0 &&
+                    ((reinterpret_cast<uintptr_t>(part) | reinterpret_cast<uintptr_t>(dx)) & 15) == 0;
+    const dim3 grid(grid_for(v4 ? n / 4 : n, 256, 1u << 20));
+    if (v4)
+        hipLaunchKernelGGL((k_splitk_rows<false, true>), grid, dim3(256), 0, st, part, dx, (int)n,
+                           make_fastdiv(1u), parts, Epi());
+    else
+        hipLaunchKernelGGL((k_splitk_rows<false, false>), grid, dim3(256), 0, st, part, dx, (int)n,
+                           make_fastdiv(1u), parts, Epi());
+    return check_launch();
 }
 
 }  // namespace ach
@@ -3409,8 +3456,11 @@ size_t ach_conv_bwd_data_workspace(const ach_conv_desc *d)
     if (g.S == 1 && g.P <= g.KS - 1) return align256(wf) + fwd_part_bytes(dgrad_as_fwd(g), false);
     // strided: the filter by phases, or one image's column buffer
     const size_t col = (size_t)g.C * g.KS * g.KS * g.OH * g.OW * sizeof(float);
-    wf = align256(wf);
-    return dgrad_phases(g) && wf > col ? wf : col;
+    if (!dgrad_phases(g)) return col;
+    const int parts = dgrad_parts(g);
+    wf = phase_filter_bytes(g) +
+         (parts > 1 ? (size_t)parts * g.B * g.C * g.H * g.W * sizeof(float) : 0);
+    return wf > col ? wf : col;
 }
 
 // bytes that ach_conv_bwd_data needs (the query adds what it makes use of)
@@ -3450,7 +3500,7 @@ int ach_conv_bwd_data(const ach_conv_desc *d, const float *dy, const float *w, f
     }
     if (!xy && dgrad_phases(g) &&
         ws_bytes >= (size_t)g.F * g.C * g.KS * g.KS * sizeof(float))
-        return dgrad_phases_launch(g, dy, w, dx, (float *)ws, st);
+        return dgrad_phases_launch(g, dy, w, dx, ws, ws_bytes, st);
     // Unequal strides, strides above PH_MAX_S or a workspace for one image's
     // columns only: the reference's per-image TN GEMM + col2im
     // (ConvolutionalLayer.c:933-945).
@@ -3627,6 +3677,8 @@ static int bwd_filter(const ach_conv_desc *d, const float *x, const float *dy, f
     if (wgrad_1x1_smallf(g) &&
         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15) == 0)
         return wgrad_1x1_smallf_launch(g, x, dy, dw, sgd, as_stream(stream));
+    if (fc_geom(g) && fc_split_wgrad(g.F, g.C, g.B))
+        return fc_split_wgrad_launch(g.F, g.C, g.B, dy, x, dw, sgd, as_stream(stream));
     const int bm = wgrad_bm(g), bn = wgrad_bn(g);
     int splits, kchunk;
     wgrad_split(g, bm, bn, splits, kchunk);

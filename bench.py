@@ -30,6 +30,9 @@ sys.path.insert(0, os.path.join(ROOT, "aet-cnn_amd"))
 sys.path.insert(0, os.path.join(ROOT, "tests"))
 
 MFMA_FP32_PEAK_TFLOPS = 157.3
+# the kernels that form a float product from six bf16 piece products: the
+# dense bf16 peak over six
+MFMA_PIECES_PEAK_TFLOPS = 2500.0 / 6
 HBM_PEAK_GBS = 8000.0
 
 SWEEP = [  # config 1: (C_in, C_out, H, k, pad)
@@ -37,17 +40,16 @@ SWEEP = [  # config 1: (C_in, C_out, H, k, pad)
     (256, 512, 8, 3, 1), (512, 512, 8, 3, 1), (512, 10, 8, 1, 0),
 ]
 # Kernel probes, each one config-1 / config-3 layer pass launched back to
-# back on its own stream: the conv forward implicit GEMM (the kernel with the
-# most time per darknet step; the stride-1 input gradient runs it too) and
-# the weight-gradient GEMM (the second most).
+# back on its own stream: the three-piece convolution (input gradients and
+# operation-level forwards run it) and the three-piece weight gradient.
 PROBES = {
     "fwd": dict(shape=(256, 256, 16, 3, 1), op="fwd",
-                kernel="k_mfma_gemm<FwdProblem<128, BIm2col3F, true, false>, 2> "
-                       "(conv fwd implicit GEMM, two K groups per workgroup; the stride-1 "
-                       "dgrad runs the same loop with one)"),
+                kernel="k_conv_split<4, 1, 1, 3, 2, false> (three-piece bf16 convolution; the "
+                       "stride-1 input gradient runs the same kernel)"),
     "wgrad": dict(shape=(128, 128, 32, 3, 1), op="wgrad",
-                  kernel="k_mfma_gemm<WgradProblemC<128, 96, 3>> (conv weight-gradient GEMM)"),
+                  kernel="k_conv_wsplit<true> (three-piece bf16 weight gradient)"),
 }
+PROBE_KERNELS = ("k_conv_split", "k_conv_wsplit")
 CALIB_FLOATS = 1 << 26  # the 256 MiB copy-calibration dispatch
 
 
@@ -301,9 +303,9 @@ def roofline_phase(aetcnn, which, batch, reps):
     """A probe launched `reps` times back to back with HIP events around the
     run on the probe's stream.  The forward call is the GEMM launch alone
     (ach_conv_fwd_prepared on a k-major filter made once: 512 workgroups of
-    two K groups over 128 x 128 tiles), so the average is that kernel's; the
-    weight-gradient call is the GEMM over chunked K and its fixed-order
-    split-K reduction (~5%), whose average is the whole call."""
+    128 x 128 tiles), so the average is that kernel's; the weight-gradient
+    call is the GEMM and its fixed-order reduction, whose average is the
+    whole call."""
     ops = aetcnn.ops()
     call, stream, free, flop, shape = probe_setup(aetcnn, which, batch)
     ms = time_launch(ops, stream, call, reps)
@@ -377,7 +379,7 @@ def traffic_phase(which, calls=3, timeout=120):
             expect_kib = CALIB_FLOATS * 4 / 1024.0
             scale[ctr] = expect_kib / disp[cal[0]][1]
             after = [i for i in ids if i > cal[0]]
-            ngemm = sum(1 for i in after if "k_mfma_gemm" in disp[i][0])
+            ngemm = sum(1 for i in after if any(k in disp[i][0] for k in PROBE_KERNELS))
             if ngemm != calls:
                 return None, f"{ctr}: expected {calls} GEMM dispatches, found {ngemm}"
             tot = 0.0
@@ -735,8 +737,8 @@ def main():
         else:
             log(f"traffic {which}: not measured ({why})")
         rooflines[which] = dict(
-            bound="mfma", achieved=round(ach, 3), peak=MFMA_FP32_PEAK_TFLOPS, unit="TFLOP/s",
-            frac=round(ach / MFMA_FP32_PEAK_TFLOPS, 4),
+            bound="mfma", achieved=round(ach, 3), peak=round(MFMA_PIECES_PEAK_TFLOPS, 1),
+            unit="TFLOP/s", frac=round(ach / MFMA_PIECES_PEAK_TFLOPS, 4),
             traffic=traffic["bytes"] if traffic else None,
             kernel=probe["kernel"], shape=probe["shape"], avg_launch_ms=round(probe["ms"], 5),
             launches=probe["reps"], flop_per_launch=probe["flop"],

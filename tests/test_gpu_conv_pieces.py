@@ -176,6 +176,7 @@ def test_weight_gradient_non_finite(gpu, value):
     (2, 16, 5, 5, 8, 3, 2, 2),       # padding 2
     (2, 4, 2, 3, 8, 2, 2, 0),        # one or two pixels per phase
     (2, 6, 7, 7, 10, 3, 5, 1),       # a stride above the phases' limit
+    (1, 36, 11, 10, 195, 5, 2, 2),   # K parts, the last phase's shorter
 ], ids=lambda s: "x".join(map(str, s)))
 def test_strided_input_gradient(gpu, shape):
     """fp32 sums of at most F*k*k products: |error| <= F k k 2^-24 sum |a||b|."""
@@ -194,3 +195,60 @@ def test_strided_input_gradient(gpu, shape):
         ws, dx = D(n // 4 + 64), D.from_numpy(np.full((B, Cc, H, W), 7.0, np.float32))
         check(gpu.ach_conv_bwd_data(C.byref(d), ddy.ptr, dw.ptr, dx.ptr, ws.ptr, n, None))
         assert np.all(abs(dx.numpy() - ref) <= F * k * k * 2.0 ** -24 * mag)
+
+
+@pytest.mark.parametrize("B,K,F", [
+    (33, 128, 128),      # two row fragments, one of them a single row; one tile
+    (64, 300, 130),      # K not a multiple of 8, ragged features
+    (65, 1024, 700),     # two 64-row fragments
+    (130, 520, 256),     # two row tiles, K slices
+    (70, 2900, 2890),    # large enough for the weight gradient's tiles
+], ids=lambda v: str(v))
+def test_fully_connected(gpu, B, K, F):
+    """Forward, input gradient and weight gradient (with and without the SGD
+    step in its pass) of a fully connected layer."""
+    rng = np.random.default_rng(B + K + F)
+    x = rng.standard_normal((B, K)).astype(np.float32)
+    w = rng.standard_normal((F, K)).astype(np.float32)
+    dy = rng.standard_normal((B, F)).astype(np.float32)
+    d = aetcnn.ConvDesc(B, K, 1, 1, F, 1, 1, 0)
+    nb = max(gpu.ach_conv_fwd_workspace(C.byref(d)), gpu.ach_conv_bwd_data_workspace(C.byref(d)),
+             gpu.ach_conv_bwd_filter_workspace(C.byref(d)))
+    ws, dx_, dw_, ddy = D(nb // 4 + 64), D.from_numpy(x), D.from_numpy(w), D.from_numpy(dy)
+    y, dx = D((B, F)), D((B, K))
+    check(gpu.ach_conv_fwd(C.byref(d), dx_.ptr, dw_.ptr, y.ptr, ws.ptr, nb, None))
+    check(gpu.ach_conv_bwd_data(C.byref(d), ddy.ptr, dw_.ptr, dx.ptr, ws.ptr, nb, None))
+    x8, w8, d8 = (a.astype(np.float64) for a in (x, w, dy))
+    for got, a, b, n in ((y, x8, w8.T, K), (dx, d8, w8, F)):
+        lim = (-(-n // 16) + 40) * 2.0 ** -24 * (abs(a) @ abs(b))
+        assert np.all(abs(got.numpy() - a @ b) <= lim)
+    v0 = rng.standard_normal((F, K)).astype(np.float32)
+    wa, va, wb, vb = (D.from_numpy(a) for a in (w, v0, w, v0))
+    dc, lc, mom = np.float32(-5e-4 * B), np.float32(0.01 / B), np.float32(0.9)
+    check(gpu.ach_conv_bwd_filter(C.byref(d), dx_.ptr, ddy.ptr, va.ptr, ws.ptr, nb, None))
+    lim = (B + 8) * 2.0 ** -24 * (abs(d8.T) @ abs(x8) + abs(v0))
+    assert np.all(abs(va.numpy() - (v0 + d8.T @ x8)) <= lim)
+    check(gpu.ach_sgd_update(w.size, wa.ptr, va.ptr, dc, lc, mom, None))
+    check(gpu.ach_conv_bwd_filter_sgd(C.byref(d), dx_.ptr, ddy.ptr, wb.ptr, vb.ptr, dc, lc, mom,
+                                      ws.ptr, nb, None))
+    assert np.array_equal(wa.numpy().view(np.uint32), wb.numpy().view(np.uint32))
+    assert np.array_equal(va.numpy().view(np.uint32), vb.numpy().view(np.uint32))
+
+
+def test_fully_connected_non_finite(gpu):
+    B, K, F = 64, 512, 256
+    rng = np.random.default_rng(1)
+    x = rng.standard_normal((B, K)).astype(np.float32)
+    w = rng.standard_normal((F, K)).astype(np.float32)
+    x[3, 100], w[17, 9] = np.inf, np.nan
+    d = aetcnn.ConvDesc(B, K, 1, 1, F, 1, 1, 0)
+    nb = gpu.ach_conv_fwd_workspace(C.byref(d))
+    ws, dx, dw, y = D(nb // 4 + 64), D.from_numpy(x), D.from_numpy(w), D((B, F))
+    check(gpu.ach_conv_fwd(C.byref(d), dx.ptr, dw.ptr, y.ptr, ws.ptr, nb, None))
+    with np.errstate(invalid="ignore"):
+        ref = x.astype(np.float64) @ w.T.astype(np.float64)
+    got = y.numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    fin = np.isfinite(ref)
+    assert np.all(abs(got[fin] - ref[fin]) <= 1e-5 * abs(ref[fin]).max())
