@@ -25,6 +25,8 @@
 // forward), so the activated tensor does not have to be re-read.
 #include "common.hpp"
 
+#include <type_traits>
+
 #include <mutex>
 
 namespace ach {
@@ -264,7 +266,7 @@ __global__ void __launch_bounds__(BN_NT) k_bn_apply(
 }
 
 // ---- forward of a small channel in one workgroup ---------------------------------
-// A channel of at most BN_CH_NT*V float4 (batch*HW <= 32768 floats: darknet's
+// A channel of at most BN_CH_NT*V float4 or floats (batch*HW <= 32768: darknet's
 // 16x16 and 8x8 layers at batch 128) is loaded once into registers, summed
 // (double: each thread's values in order, then the block's fixed tree) and
 // normalized from the registers: one read and one write of the tensor in one
@@ -274,25 +276,36 @@ __global__ void __launch_bounds__(BN_NT) k_bn_apply(
 // may be out (every thread writes only what it read, after the block's
 // barrier); xcopy / xnorm optional as in k_bn_apply.
 constexpr int BN_CH_NT = 1024;
+// Tensors of at most BN_ONE_LAUNCH values in channels of at most BN_ONE_CH take
+// one launch per direction whatever their channel count: forward 9-10 -> 5.5-7
+// us, backward 12-17 -> 7-10 us over shapes from 54 K to 1 M values (channels
+// of 441 to 16384); with 32768 values a channel's one workgroup is slower
+// (forward 10.5 against 9.6 us, backward 15.9 against 14.2).
+constexpr long long BN_ONE_LAUNCH = 1ll << 20, BN_ONE_CH = 16384;
+static bool bn_one_launch(int batch, int c, int hw)
+{
+    return (long long)batch * hw <= BN_ONE_CH && (long long)batch * c * hw <= BN_ONE_LAUNCH;
+}
 constexpr int BN_CH_MAXV = 8;  // float4 per thread
-template <int V>
+template <int V, bool VEC>
 __global__ void __launch_bounds__(BN_CH_NT) k_bn_fwd_channel(
-    const float *src, float *xcopy, float *xnorm, float *out, int batch, int C, int HW, int hw4,
+    const float *src, float *xcopy, float *xnorm, float *out, int batch, int C, int HW, int hwv,
     float *__restrict__ mean, float *__restrict__ variance, float *__restrict__ rmean,
     float *__restrict__ rvar, const float *__restrict__ scales, const float *__restrict__ biases,
     int act)
 {
+    typedef typename Elem<VEC>::T T;
     __shared__ double sh[BN_CH_NT / 64];
     __shared__ float sp[2];
-    const int c = blockIdx.x, tot = batch * hw4;
-    const float4 *s4 = reinterpret_cast<const float4 *>(src);
-    float4 v[V];
+    const int c = blockIdx.x, tot = batch * hwv;
+    const T *s4 = reinterpret_cast<const T *>(src);
+    T v[V];
     int at[V];
     double s1 = 0, s2 = 0;
 #pragma unroll
     for (int u = 0; u < V; ++u) {
-        const int e = threadIdx.x + u * BN_CH_NT, b = e / hw4;
-        at[u] = e < tot ? (b * C + c) * hw4 + (e - b * hw4) : -1;
+        const int e = threadIdx.x + u * BN_CH_NT, b = e / hwv;
+        at[u] = e < tot ? (b * C + c) * hwv + (e - b * hwv) : -1;
     }
 #pragma unroll
     for (int u = 0; u < V; ++u)
@@ -301,7 +314,7 @@ __global__ void __launch_bounds__(BN_CH_NT) k_bn_fwd_channel(
     for (int u = 0; u < V; ++u) {
         if (at[u] < 0) continue;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
+        for (int k = 0; k < Elem<VEC>::N; ++k) {
             const float e = comp(v[u], k);
             s1 += (double)e;
             s2 += (double)(e * e);
@@ -326,17 +339,17 @@ __global__ void __launch_bounds__(BN_CH_NT) k_bn_fwd_channel(
     }
     __syncthreads();
     const float mu = sp[0], iv = sp[1], sc = scales[c], bb = biases[c];
-    float4 *o4 = reinterpret_cast<float4 *>(out);
+    T *o4 = reinterpret_cast<T *>(out);
 #pragma unroll
     for (int u = 0; u < V; ++u) {
         if (at[u] < 0) continue;
-        if (xcopy) reinterpret_cast<float4 *>(xcopy)[at[u]] = v[u];
-        float4 n, o;
+        if (xcopy) reinterpret_cast<T *>(xcopy)[at[u]] = v[u];
+        T n, o;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) comp(n, k) = (comp(v[u], k) - mu) * iv;
-        if (xnorm) reinterpret_cast<float4 *>(xnorm)[at[u]] = n;
+        for (int k = 0; k < Elem<VEC>::N; ++k) comp(n, k) = (comp(v[u], k) - mu) * iv;
+        if (xnorm) reinterpret_cast<T *>(xnorm)[at[u]] = n;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) comp(o, k) = act_forward(__fmaf_rn(comp(n, k), sc, bb), act);
+        for (int k = 0; k < Elem<VEC>::N; ++k) comp(o, k) = act_forward(__fmaf_rn(comp(n, k), sc, bb), act);
         o4[at[u]] = o;
     }
 }
@@ -499,6 +512,91 @@ __global__ void __launch_bounds__(BN_NT) k_bn_bwd_apply(
     }
 }
 
+// The backward of a small channel in one launch: one workgroup per channel
+// holds its x and delta in registers, reduces (each thread's values in order,
+// then the block's fixed tree, in double) and writes from the registers, with
+// the arithmetic of the two passes above.  Bound: latency; it replaces two
+// dependent launches where the tensor is too small to need the chip (72
+// channels of 4560 values: 12.1 -> 8.5 us a call).
+template <int V, bool VEC>
+__global__ void __launch_bounds__(BN_CH_NT) k_bn_bwd_channel(
+    float *__restrict__ delta, const float *__restrict__ x, int batch, int C, int HW, int hwv,
+    const float *__restrict__ mean, const float *__restrict__ variance,
+    const float *__restrict__ scales, const float *__restrict__ biases, int act,
+    float *__restrict__ scale_updates, float *__restrict__ mean_delta,
+    float *__restrict__ variance_delta)
+{
+    typedef typename Elem<VEC>::T T;
+    __shared__ double sh[BN_CH_NT / 64];
+    __shared__ double coef[3];
+    const int c = blockIdx.x, tot = batch * hwv;
+    T xv[V], dv[V];
+    int at[V];
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        const int e = threadIdx.x + u * BN_CH_NT, b = e / hwv;
+        at[u] = e < tot ? (b * C + c) * hwv + (e - b * hwv) : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < V; ++u)
+        if (at[u] >= 0) {
+            xv[u] = reinterpret_cast<const T *>(x)[at[u]];
+            dv[u] = reinterpret_cast<const T *>(delta)[at[u]];
+        }
+    const float ve0 = variance[c], mu = mean[c], iv = bn_inv(ve0), s = scales[c];
+    const float bb = biases ? biases[c] : 0.f;
+    double g1 = 0, g2 = 0, g3 = 0;
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        if (at[u] < 0) continue;
+#pragma unroll
+        for (int k = 0; k < Elem<VEC>::N; ++k) {
+            const float xe = comp(xv[u], k);
+            const float g = bwd_grad(comp(dv[u], k), xe, mu, iv, s, bb, act);
+            const float gs = g * s;
+            comp(dv[u], k) = gs;
+            g1 += (double)(g * ((xe - mu) * iv));
+            g2 += (double)gs;
+            g3 += (double)(gs * (xe - mu));
+        }
+    }
+    const double G1 = block_sum<BN_CH_NT / 64>(g1, sh);
+    const double G2 = block_sum<BN_CH_NT / 64>(g2, sh);
+    const double G3 = block_sum<BN_CH_NT / 64>(g3, sh);
+    if (threadIdx.x == 0) {
+        const int N = batch * HW;
+        const float ve = ve0 + 1e-5f;
+        const float md = (float)((double)(float)G2 * (-1. / sqrt((double)ve)));
+        const float vd = (float)((double)(float)G3 * (-.5 * pow((double)ve, (double)(-1.5f))));
+        scale_updates[c] += (float)G1;
+        if (mean_delta) mean_delta[c] = md;
+        if (variance_delta) variance_delta[c] = vd;
+        coef[0] = 1. / sqrt((double)ve);
+        coef[1] = (double)vd * 2. / (double)N;
+        coef[2] = (double)(md / (float)N);
+    }
+    __syncthreads();
+    const double k0 = coef[0], k1 = coef[1], k2 = coef[2];
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        if (at[u] < 0) continue;
+        T o;
+#pragma unroll
+        for (int k = 0; k < Elem<VEC>::N; ++k)
+            comp(o, k) = (float)((double)comp(dv[u], k) * k0 + k1 * (double)(comp(xv[u], k) - mu) + k2);
+        reinterpret_cast<T *>(delta)[at[u]] = o;
+    }
+}
+
+// Values (float4 or float) per thread of the one-workgroup kernels, 0 where a
+// channel does not fit
+static int bn_channel_v(long long per_channel, bool vec)
+{
+    for (int v = 1; v <= (vec ? BN_CH_MAXV : 2 * BN_CH_MAXV); v *= 2)
+        if (per_channel <= (long long)v * BN_CH_NT) return v;
+    return 0;
+}
+
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 static size_t bn_ws_bytes(int batch, int c)
@@ -543,6 +641,26 @@ static BnPlan bn_plan(int batch, int C, int HW, bool vec_ok, int apply_blocks,
     return p;
 }
 
+// f(V, VEC) of the one-workgroup-per-channel kernels
+template <class Fn>
+static int bn_dispatch(int V, bool vec, Fn f)
+{
+    using std::integral_constant;
+    using std::true_type;
+    using std::false_type;
+    if (vec) {
+        if (V == 1) return f(integral_constant<int, 1>(), true_type());
+        if (V == 2) return f(integral_constant<int, 2>(), true_type());
+        if (V == 4) return f(integral_constant<int, 4>(), true_type());
+        return f(integral_constant<int, 8>(), true_type());
+    }
+    if (V == 1) return f(integral_constant<int, 1>(), false_type());
+    if (V == 2) return f(integral_constant<int, 2>(), false_type());
+    if (V == 4) return f(integral_constant<int, 4>(), false_type());
+    if (V == 8) return f(integral_constant<int, 8>(), false_type());
+    return f(integral_constant<int, 16>(), false_type());
+}
+
 static int bn_fwd(const float *src, float *xcopy, float *xnorm, float *out, int batch, int C,
                   int HW, const float *scales, const float *biases, float *mean,
                   float *variance, float *rmean, float *rvar, int act, void *ws,
@@ -557,18 +675,19 @@ static int bn_fwd(const float *src, float *xcopy, float *xnorm, float *out, int 
                              aligned16(src) && aligned16(out) && aligned16(xcopy) &&
                                  aligned16(xnorm),
                              BN_FWD_APPLY_BLOCKS, BN_FWD_RED_BLOCKS);
-    // one workgroup per channel when the channel fits its registers and the
-    // channels alone give about a workgroup per CU
-    const long long ch4 = (long long)batch * p.hwv;
-    if (p.vec && C >= 128 && ch4 <= (long long)BN_CH_NT * BN_CH_MAXV) {
-        const int V = ch4 <= BN_CH_NT ? 1 : (ch4 <= 2 * BN_CH_NT ? 2 : (ch4 <= 4 * BN_CH_NT ? 4 : 8));
-        void (*kern)(const float *, float *, float *, float *, int, int, int, int, float *, float *,
-                     float *, float *, const float *, const float *, int) =
-            V == 1 ? k_bn_fwd_channel<1>
-                   : (V == 2 ? k_bn_fwd_channel<2> : (V == 4 ? k_bn_fwd_channel<4> : k_bn_fwd_channel<8>));
-        hipLaunchKernelGGL(kern, dim3(C), dim3(BN_CH_NT), 0, st, src, xcopy, xnorm, out, batch, C,
-                           HW, p.hwv, mean, variance, rmean, rvar, scales, biases, act);
-        return check_launch();
+    // one workgroup per channel when the channel fits its registers and either
+    // the channels alone give about a workgroup per CU, or the tensor is too
+    // small for two launches to pay
+    const long long ch = (long long)batch * p.hwv;
+    const int V = bn_channel_v(ch, p.vec);
+    if (V && ((p.vec && C >= 128) || bn_one_launch(batch, C, HW))) {
+        auto go = [&](auto v, auto vec) {
+            hipLaunchKernelGGL((k_bn_fwd_channel<decltype(v)::value, decltype(vec)::value>), dim3(C),
+                               dim3(BN_CH_NT), 0, st, src, xcopy, xnorm, out, batch, C, HW, p.hwv,
+                               mean, variance, rmean, rvar, scales, biases, act);
+            return check_launch();
+        };
+        return bn_dispatch(V, p.vec, go);
     }
     if (p.vec)
         hipLaunchKernelGGL(k_bn_stats<true>, p.reduce_grid, dim3(BN_NT), 0, st, src, batch, C,
@@ -738,6 +857,16 @@ int ach_bn_bwd(float *delta, int batch, int C, int HW, const float *x, const flo
     const BnPlan p = bn_plan(batch, C, HW, aligned16(delta) && aligned16(x) && aligned16(x_norm),
                              BN_BWD_APPLY_BLOCKS, small ? BN_FWD_RED_BLOCKS : BN_BWD_RED_BLOCKS);
     const int act = fused ? activation : ACH_LINEAR;
+    const int V = bn_channel_v((long long)batch * p.hwv, p.vec);
+    if (V && !x_norm && bn_one_launch(batch, C, HW)) {
+        auto go = [&](auto v, auto vec) {
+            hipLaunchKernelGGL((k_bn_bwd_channel<decltype(v)::value, decltype(vec)::value>), dim3(C),
+                               dim3(BN_CH_NT), 0, st, delta, x, batch, C, HW, p.hwv, mean, variance,
+                               scales, biases, act, scale_updates, mean_delta, variance_delta);
+            return check_launch();
+        };
+        return bn_dispatch(V, p.vec, go);
+    }
     if (p.vec)
         hipLaunchKernelGGL(k_bn_bwd_reduce<true>, p.reduce_grid, dim3(BN_NT), 0, st, delta, x,
                            x_norm, batch, C, p.hwv, p.per, mean, variance, scales, biases, act,
