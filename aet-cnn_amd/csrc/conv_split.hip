@@ -11,8 +11,9 @@
 // product, and runs 16 times its rate, so the six passes cost 6/16 of the
 // fp32 instruction's matrix time.
 //
-// Non-finite values: an infinity (or a finite value that rounds to one in
-// bf16) leaves NaN residuals, so the tile's sums come out non-finite; a wave
+// Non-finite values: an infinity (or a finite value above 2^103, which the
+// operands' scale of 2^24 takes to one) leaves non-finite residuals, so the
+// tile's sums come out non-finite; a wave
 // that finds a non-finite sum recomputes its tile in plain fp32, which gives
 // the infinities and NaNs of fp32 arithmetic.
 //
@@ -303,6 +304,11 @@ __global__ void __launch_bounds__(64 * WM * WN * KG, 2) k_conv_split(SplitFwd p)
                 }
             hi[f] = s;
         }
+    } else {
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) hi[f][r] *= kSumDown;
     }
     // each group hands the other the half of the fragments that one stores
     if constexpr (KG == 2) {

@@ -134,7 +134,7 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
         for (int q = 0; q < 3; ++q) *reinterpret_cast<v4u *>(dst + q * 2 * R * 16) = pc[q];
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const float a = r[8 + 2 * i], b = r[9 + 2 * i];
+            const float a = r[8 + 2 * i] * kPieceUp, b = r[9 + 2 * i] * kPieceUp;
             const unsigned h = pk_bf16(a, b);
             const float ra = a - bf_lo(h), rb = b - bf_hi(h);
             const unsigned m = pk_bf16(ra, rb);
@@ -269,6 +269,11 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
             }
             acc[q / KS][q % KS] = a;
         }
+    } else {
+#pragma unroll
+        for (int q = 0; q < T; ++q)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[q / KS][q % KS][e] *= kSumDown;
     }
     // the groups exchange tiles in rounds of QR taps: group q & 1 stores tap q
     constexpr int QR = 4;

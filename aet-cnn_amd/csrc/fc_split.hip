@@ -190,6 +190,13 @@ __global__ void __launch_bounds__(256, 2) k_fc_split(FcSplit p)
                 }
                 hi[i][j] = s;
             }
+    } else {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) hi[i][j][e] *= kSumDown;
     }
 #pragma unroll
     for (int i = 0; i < MT; ++i)

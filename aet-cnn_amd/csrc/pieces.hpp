@@ -20,12 +20,21 @@ __device__ __forceinline__ unsigned pk_bf16(float a, float b)
 __device__ __forceinline__ float bf_lo(unsigned u) { return __uint_as_float(u << 16); }
 __device__ __forceinline__ float bf_hi(unsigned u) { return __uint_as_float(u & 0xffff0000u); }
 
-// eight floats -> three pieces of eight bf16 (f = p[0] + p[1] + p[2] exactly)
+// Operands are split as kPieceUp * f: the last bit of any float, subnormals
+// included, is then at least 2^-125, so no piece is below bf16's normal range
+// (unscaled, the pieces of values under 2^-110 lost bits: 2.6e-6 instead of
+// 4e-7 from 64 bits at 1e-35, 2.6e-4 at 1e-37; scaled 1.4e-7 at any magnitude).
+// Sums of products are taken back with kSumDown, exact but for a result that
+// is subnormal itself.  Values above 2^103 and sums above 2^80 come out
+// non-finite and take the fp32 recomputation.
+constexpr float kPieceUp = 0x1p24f, kSumDown = 0x1p-48f;
+
+// eight floats -> three pieces of eight bf16 (kPieceUp * f = p[0] + p[1] + p[2] exactly)
 __device__ __forceinline__ void split8(const float *f, v4u *p)
 {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const float a = f[2 * i], b = f[2 * i + 1];
+        const float a = f[2 * i] * kPieceUp, b = f[2 * i + 1] * kPieceUp;
         const unsigned h = pk_bf16(a, b);
         const float ra = a - bf_lo(h), rb = b - bf_hi(h);
         const unsigned m = pk_bf16(ra, rb);

@@ -97,6 +97,44 @@ def test_non_finite_and_largest_values(gpu, shape, value):
     assert np.all(abs(a[fin] - b[fin]) <= 1e-5 * abs(b[fin]) + 1e-5 * abs(b[near]).max())
 
 
+# magnitudes (input, filter): inputs with subnormals among them, filters near
+# the largest float, inputs whose pieces would be below bf16's normal range
+SCALES = [(1e-37, 1e10), (1e-38, 1e20), (1e30, 1e-36), (1e-35, 1.0)]
+
+
+@pytest.mark.parametrize("sx,sw", SCALES, ids=str)
+def test_extreme_magnitudes(gpu, sx, sw):
+    """The bounds of ordinary magnitudes hold over the floats' whole range."""
+    rng = np.random.default_rng(11)
+
+    def draw(scale, *shape):
+        return (rng.standard_normal(shape) * scale).astype(np.float32)
+
+    B, Cc, H, W, F, k, p = 8, 64, 8, 8, 64, 3, 1
+    x, w = draw(sx, B, Cc, H, W), draw(sw, F, Cc, k, k)
+    d = aetcnn.ConvDesc(B, Cc, H, W, F, k, 1, p)
+    nb = gpu.ach_conv_fwd_workspace(C.byref(d))
+    ws, dx, dw, y = D(nb // 4 + 64), D.from_numpy(x), D.from_numpy(w), D((B, F, H, W))
+    check(gpu.ach_conv_fwd(C.byref(d), dx.ptr, dw.ptr, y.ptr, ws.ptr, nb, None))
+    ref, mag = refs64.conv_ref(x, w, 1, p), refs64.conv_ref(abs(x), abs(w), 1, p)
+    assert np.all(abs(y.numpy() - ref) <= bound(mag, k, Cc))
+    B, Cc, H, W, F = WGRAD[0]
+    x, dy = draw(sx, B, Cc, H, W), draw(sw, B, F, H, W)
+    got = run_wgrad(gpu, x, dy, np.zeros((F, Cc, 3, 3), np.float32)).astype(np.float64)
+    x, dy = x.astype(np.float64), dy.astype(np.float64)
+    size = np.sqrt(wgrad_ref(x * x, dy * dy))
+    n = 6 * B * H * -(-W // 8) / 2 + 64
+    assert np.all(abs(got - wgrad_ref(x, dy)) <= 8 * n ** 0.5 * 2.0 ** -25 * size)
+    B, K, F = 64, 512, 256
+    x, w = draw(sx, B, K), draw(sw, F, K)
+    d = aetcnn.ConvDesc(B, K, 1, 1, F, 1, 1, 0)
+    nb = gpu.ach_conv_fwd_workspace(C.byref(d))
+    ws, dx, dw, y = D(nb // 4 + 64), D.from_numpy(x), D.from_numpy(w), D((B, F))
+    check(gpu.ach_conv_fwd(C.byref(d), dx.ptr, dw.ptr, y.ptr, ws.ptr, nb, None))
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    assert np.all(abs(y.numpy() - x @ w.T) <= (K // 16 + 40) * 2.0 ** -24 * (abs(x) @ abs(w.T)))
+
+
 # shapes large enough for the three-piece weight gradient
 WGRAD = [
     (32, 512, 8, 8, 512),     # one segment per row: image pairs
