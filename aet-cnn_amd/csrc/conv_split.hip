@@ -410,22 +410,24 @@ SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, int fp32_splits, int 
     const int nchunk = (g.C + SP_CH - 1) / SP_CH, nt = (N + SP_BN - 1) / SP_BN;
     const int wide = M <= 32 ? 1 : (M <= 64 ? 2 : (M <= 96 ? 3 : 4));
     const long long big = (long long)((M + 127) / 128) * nt;  // 128 x 128 tiles
-    // Waves along M and K parts: the modelled time (us) of the rounds of
-    // workgroups, two per CU (or one with two K groups), plus the split-K
-    // reduction.  Measured: 11 us per 16-channel chunk of a 3x3 filter with
-    // two 128 x 128 workgroups on every CU (128 -> 128 @ 32x32, batch 128),
-    // 0.65 of it with one; tiles of half and a quarter of the fragments per
-    // wave take 6.2 and 3.6 (every wave loads the filter rows again), down to
-    // about 2.2 us for the loads' latency, and win where the grid is small
-    // (a 13-layer net's inference of one image: 227 -> 201 us).  Small grids take no more slices than the fp32 plan.
+    // Waves along M and K parts: the modelled time of the rounds of workgroups,
+    // two per CU (or one with two K groups), plus the split-K reduction.  us per
+    // 16-channel chunk of a 3x3 filter with two workgroups on every CU and with
+    // one, by waves along M, fitted to a sweep of 30 layers that ran each height
+    // in turn (one wave's 32 rows: every wave loads the filter rows again).
+    // Against fixed prices of 11 / 6.2 / 3.6 us for 3-4 / 2 / 1 waves: 256 -> 96
+    // 5x5 at 27x27, batch 128: 692 -> 555 us; 128 -> 128 at 32x32, batch 40:
+    // 88 -> 72.  Small grids take no more slices than the fp32 plan.
+    static const double kPaired[5] = {0, 4.1, 5.8, 8.0, 10.6};
+    static const double kSingle[5] = {0, 2.5, 3.5, 5.2, 7.0};
     double best = -1;
     for (int wm = wide; wm >= 1; wm = wm == 4 ? 2 : wm - 1) {
         const int wn = wm == 1 ? 4 : (wm == 2 ? 2 : 1), thr = 64 * wm * wn;
         const long long tpt = (2 * nreal + thr - 1) / thr;
         const long long tiles = (long long)((M + 32 * wm - 1) / (32 * wm)) * nt;
         if (tpt > 4 || tiles > 0x7fffffffLL) continue;
-        const double per9 = wn == 1 ? 11.0 : (wn == 2 ? 6.2 : 3.6), taps = g.KS * g.KS / 9.0;
-        const double paired = per9 * taps, single = (per9 * 0.65 > 2.2 ? per9 * 0.65 : 2.2) * taps;
+        const double taps = g.KS * g.KS / 9.0;
+        const double paired = kPaired[wm] * taps, single = kSingle[wm] * taps;
         for (int kg = 1; kg <= (kg_ok && wm == 4 && tpt <= 3 ? 2 : 1); ++kg)
             for (const int s : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 24, 32}) {
                 if (s * kg > nchunk || (s > 1 && tiles * s > 2048)) break;
