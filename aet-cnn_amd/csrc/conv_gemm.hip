@@ -3677,14 +3677,14 @@ static int bwd_filter(const ach_conv_desc *d, const float *x, const float *dy, f
     if (wgrad_1x1_smallf(g) &&
         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15) == 0)
         return wgrad_1x1_smallf_launch(g, x, dy, dw, sgd, as_stream(stream));
-    if (fc_geom(g) && fc_split_wgrad(g.F, g.C, g.B))
-        return fc_split_wgrad_launch(g.F, g.C, g.B, dy, x, dw, sgd, as_stream(stream));
     const int bm = wgrad_bm(g), bn = wgrad_bn(g);
     int splits, kchunk;
     wgrad_split(g, bm, bn, splits, kchunk);
     const size_t need = fp32_wgrad_bytes(g);
     if (need && (!ws || ws_bytes < need)) return ACH_EWORKSPACE;
     hipStream_t st = as_stream(stream);
+    if (fc_geom(g) && fc_split_wgrad(g.F, g.C, g.B))
+        return fc_split_wgrad_launch(g.F, g.C, g.B, dy, x, dw, sgd, st);
     float *part = (float *)ws;
     int rc;
     bool done = false;  // the update was applied in the GEMM's epilogue
