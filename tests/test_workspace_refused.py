@@ -12,7 +12,7 @@ ACH_EWORKSPACE = -2
 @pytest.mark.parametrize("dims", [
     (128, 4096, 1, 1, 4096, 1, 0),   # fully connected, three-piece tiles
     (128, 256, 4, 4, 3000, 4, 0),    # the same behind a plane
-    (48, 4096, 1, 1, 4096, 1, 0),    # fully connected, fp32 kernels
+    (128, 512, 1, 1, 512, 1, 0),     # fully connected, fp32 kernels
     (32, 512, 8, 8, 512, 3, 1),      # 3x3, three-piece tiles
 ], ids=lambda d: "x".join(map(str, d)))
 def test_weight_gradient_needs_its_workspace(dims):
