@@ -469,11 +469,9 @@ static int split_go(const SplitFwd &p, const SplitFwdPlan &pl, hipStream_t st)
     auto kern = epi ? &k_conv_split<WM, WN, KG, KS, TPT, true>
                     : &k_conv_split<WM, WN, KG, KS, TPT, false>;
     if (lds > 64 * 1024) {
-        // (the limit, not this launch's size: another thread may be between
-        // the two calls with the same kernel and other sizes)
         const int rc = check(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 160 * 1024));
+                                                 (int)lds));
         if (rc) return rc;
     }
     hipLaunchKernelGGL(kern, dim3(p.tiles, p.splits), dim3(64 * WM * WN * KG), lds, st, p);
