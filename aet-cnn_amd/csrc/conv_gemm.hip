@@ -976,33 +976,46 @@ struct FwdProblem {
 // of the input meets only the taps ki = ra + S*ti with ra = (a + P) mod S
 // (kj likewise), at output row i + (a + P - ra)/S - ti: every phase (a, b) is
 // a stride-1 convolution of dy with its own taps, so no product is with a
-// zero.  All phases run in one launch, a grid slice each:
-//   dx[b][c][S*i+a][S*j+b] = sum over (f, ti, tj) Wp[k][c] * dy[b][f][oh][ow]
-// with Wp the filter regrouped k-major by phase (k_phase_filters).  A phase
-// without taps (a window narrower than the stride) stores zeros.
+// zero between strided pixels.  All phases run in one launch, a grid slice
+// each:
+//   dx[b][c][S*i+a][S*j+b] = sum over (ti, tj) of (sum over f of
+//                            Wp[k][c] * dy[b][f][oh][ow])
+// with Wp the filter regrouped k-major by phase and tap (k_phase_filters),
+// each tap's filters padded with zero rows to whole k-tiles.  A phase without
+// taps (a window narrower than the stride) stores zeros.
+// The sums are those of the reference's GEMM and col2im: a tap's sum over the
+// filters is finished by itself and added where its row and column of dy
+// exist (tap_end, tap_valid).  A tap beyond dy's edge so adds nothing, an
+// infinite or NaN weight included (as a product with a zero it would add a
+// NaN), and the error is that of the short sums: in one chain over filters and
+// taps it was 1.3 to 2.5 times larger (32 -> 64 channels 5x5 stride 2 at 64x64,
+// batch 16: 3.7e-7 instead of 1.5e-7 from 64 bits).
 // Bound: fp32 MFMA and the launch.  It replaces a GEMM and a col2im launch
 // per image: 72 -> 48 channels at 37x29, stride 2, batch 16: the layer's training pass 461 -> 90 us.
 constexpr int PH_MAX_S = 4;
+constexpr int PH_BK = 16;  // k-tile; a tap's filters are padded to a multiple
 struct Phase {
     int k0, nk;        // its rows of Wp
     int h, w, n;       // its pixels per image, B*h*w
     int oy, ox;        // output row of pixel row 0 at tap 0
     int a, b, tb;      // phase, taps along the width
     int ra, rb;        // first tap
-    FastDiv dt, dtb, dhw, dw;
+    FastDiv dtb, dhw, dw;
 };
 struct PhaseTable {
     Phase p[PH_MAX_S * PH_MAX_S];
     int n;
+    int fp;            // rows of Wp per tap: F padded to whole k-tiles
+    FastDiv dfp;
 };
 
 struct BPhase {
-    static constexpr int BK = 16, RB = 8, PAD = LDP_FWD;
+    static constexpr int BK = PH_BK, RB = 8, PAD = LDP_FWD;
     __amdgpu_buffer_rsrc_t rs;
-    int base, i, j, kr, ok, OH, OW, nt, tb, k0;
-    FastDiv dt, dtb;
-    __device__ __forceinline__ void init(const float *dy, const ConvGeom &g, const Phase &ph, int n0,
-                                         int tid)
+    int base, i, j, kr, ok, OH, OW, F, tb, k0, fp;
+    FastDiv dfp, dtb;
+    __device__ __forceinline__ void init(const float *dy, const ConvGeom &g, const PhaseTable &t,
+                                         const Phase &ph, int n0, int tid)
     {
         rs = make_rsrc(dy, (unsigned)((size_t)g.B * g.F * g.OH * g.OW * 4));
         const int n = n0 + tid % GBN;
@@ -1013,24 +1026,27 @@ struct BPhase {
         const int r = fdiv(p, ph.dw), c = p - r * ph.w;
         OH = g.OH;
         OW = g.OW;
+        F = g.F;
         base = b * g.F * g.OH * g.OW;
         i = r + ph.oy;
         j = c + ph.ox;
-        nt = (int)ph.dt.d;
         tb = ph.tb;
         k0 = ph.k0;
-        dt = ph.dt;
+        fp = t.fp;
+        dfp = t.dfp;
         dtb = ph.dtb;
     }
+    // (a k-tile lies within one tap)
     __device__ __forceinline__ void load(int kt, int ke, float *rv) const
     {
+        const int kk = kt - k0, t = fdiv(kk, dfp), f0 = kk - t * fp + kr;
+        const int ti = fdiv(t, dtb), oh = i - ti, ow = j - (t - ti * tb);
+        const bool v = ok && kt < ke && (unsigned)oh < (unsigned)OH && (unsigned)ow < (unsigned)OW;
+        const int at = base + oh * OW + ow;
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            const int kk = kt + kr + 2 * q, k = kk - k0;
-            const int f = fdiv(k, dt), t = k - f * nt, ti = fdiv(t, dtb), tj = t - ti * tb;
-            const int oh = i - ti, ow = j - tj;
-            const bool v = ok && kk < ke && (unsigned)oh < (unsigned)OH && (unsigned)ow < (unsigned)OW;
-            rv[q] = bload(rs, boff(v, base + (f * OH + oh) * OW + ow));
+            const int f = f0 + 2 * q;
+            rv[q] = bload(rs, boff(v && f < F, at + f * OH * OW));
         }
     }
     template <int LD>
@@ -1053,7 +1069,7 @@ struct DgradPhase {
     ConvGeom g;
     int M, K, parts;
     PhaseTable tab;
-    // grid slice z: part z % parts of phase z / parts
+    // grid slice z: part z % parts of phase z / parts, whole k-tiles
     __device__ __forceinline__ void krange(int z, int &kb, int &ke) const
     {
         const Phase &ph = tab.p[z / parts];
@@ -1066,7 +1082,25 @@ struct DgradPhase {
     {
         int z = 0;  // (a phase without rows never loads)
         while (z + 1 < tab.n && !(tab.p[z].k0 <= kb && kb < tab.p[z].k0 + tab.p[z].nk)) ++z;
-        b.init(dy, g, tab.p[z], n0, tid);
+        b.init(dy, g, tab, tab.p[z], n0, tid);
+    }
+    // whether the rows up to k (a multiple of BK after the phase's first)
+    // finish a tap
+    __device__ __forceinline__ bool tap_end(int z, int k) const
+    {
+        const int kk = k - tab.p[z / parts].k0;
+        return fdiv(kk, tab.dfp) * tab.fp == kk;
+    }
+    // whether pixel n meets an output at the tap of row k
+    __device__ __forceinline__ bool tap_valid(int z, int k, int n) const
+    {
+        const Phase &ph = tab.p[z / parts];
+        const int t = fdiv(k - ph.k0, tab.dfp), ti = fdiv(t, ph.dtb);
+        const int nn = n < ph.n ? n : 0;
+        const int b = fdiv(nn, ph.dhw), p = nn - b * ph.h * ph.w;
+        const int r = fdiv(p, ph.dw), c = p - r * ph.w;
+        return (unsigned)(r + ph.oy - ti) < (unsigned)g.OH &&
+               (unsigned)(c + ph.ox - (t - ti * ph.tb)) < (unsigned)g.OW;
     }
     __device__ __forceinline__ void store_tile(int mb, int n, const v16f &acc, int z, bool) const
     {
@@ -1084,11 +1118,12 @@ struct DgradPhase {
     }
 };
 
-// Wp[k][c] = w[f][c][ra + S*ti][rb + S*tj], k = k0 + f*taps + ti*tb + tj of
-// each phase; one block per 256 values, coalesced along c
+// Wp[k][c] = w[f][c][ra + S*ti][rb + S*tj], k = k0 + (ti*tb + tj)*fp + f of
+// each phase (0 for F <= f < fp); one block per 256 values, stored coalesced
+// along c
 __global__ void __launch_bounds__(256) k_phase_filters(const float *__restrict__ w,
-                                                       float *__restrict__ wp, int C, int KS, int S,
-                                                       int total, FastDiv dc, PhaseTable tab)
+                                                       float *__restrict__ wp, int C, int F, int KS,
+                                                       int S, int total, FastDiv dc, PhaseTable tab)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= total) return;
@@ -1096,9 +1131,9 @@ __global__ void __launch_bounds__(256) k_phase_filters(const float *__restrict__
     int z = 0;
     while (z + 1 < tab.n && !(k < tab.p[z].k0 + tab.p[z].nk)) ++z;
     const Phase &ph = tab.p[z];
-    const int kk = k - ph.k0, f = fdiv(kk, ph.dt), t = kk - f * (int)ph.dt.d;
+    const int kk = k - ph.k0, t = fdiv(kk, tab.dfp), f = kk - t * tab.fp;
     const int ti = fdiv(t, ph.dtb), tj = t - ti * ph.tb;
-    wp[i] = w[(((size_t)f * C + c) * KS + ph.ra + S * ti) * KS + ph.rb + S * tj];
+    wp[i] = f < F ? w[(((size_t)f * C + c) * KS + ph.ra + S * ti) * KS + ph.rb + S * tj] : 0.f;
 }
 
 // dW tile stores of the weight-gradient problems (dw[m][n] row-major, one
@@ -1371,6 +1406,11 @@ struct odd_last_k<P, std::void_t<decltype(P::ODD_K)>> : std::bool_constant<P::OD
 template <class P, class = void> struct early_b_store : std::false_type {};
 template <class P>
 struct early_b_store<P, std::void_t<decltype(P::EARLY_B)>> : std::bool_constant<P::EARLY_B> {};
+// problems that finish the sum of each tap by itself (tap_end, tap_valid)
+template <class P, class = void> struct sums_by_tap : std::false_type {};
+template <class P>
+struct sums_by_tap<P, std::void_t<decltype(std::declval<const P &>().tap_end(0, 0))>>
+    : std::true_type {};
 template <class P, class = void> struct WavesPerEU { static constexpr int v = 1; };
 template <class P> struct WavesPerEU<P, std::void_t<decltype(P::kWPE)>> {
     static constexpr int v = P::kWPE;
@@ -1494,6 +1534,14 @@ k_mfma_gemm(P p, int mt, int nt)
     for (int i = 0; i < (ODD_COLS ? TM : 1); ++i)
 #pragma unroll
         for (int r = 0; r < 32; ++r) accw[i][r] = 0.f;
+    constexpr bool BY_TAP = sums_by_tap<P>::value;
+    v16f sum[BY_TAP ? TM : 1][BY_TAP ? TN : 1];
+#pragma unroll
+    for (int i = 0; i < (BY_TAP ? TM : 1); ++i)
+#pragma unroll
+        for (int j = 0; j < (BY_TAP ? TN : 1); ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sum[i][j][r] = 0.f;
     for (int kt = 0; kt < nkt; ++kt) {
         const int cur = kt & 1;
         // next k-tile (past ke on the last tile: the loaders read zeros or
@@ -1584,6 +1632,27 @@ k_mfma_gemm(P p, int mt, int nt)
             }
         }
         __syncthreads();
+        if constexpr (BY_TAP) {
+            if (p.tap_end(z, k0n) || kt + 1 == nkt) {
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const bool v = p.tap_valid(z, k0n - BK, n0 + (j * WN + wn) * 32 + lcol);
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            sum[i][j][r] += v ? acc[i][j][r] : 0.f;
+                            acc[i][j][r] = 0.f;
+                        }
+                }
+            }
+        }
+    }
+    if constexpr (BY_TAP) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = sum[i][j];
     }
     if constexpr (ODD_COLS) {
 #pragma unroll
@@ -3296,14 +3365,18 @@ static int dgrad_small_c_launch(const ConvGeom &g, const float *dy, const float 
 // (and images whose own GEMM, k*k*C x OH*OW, fills the chip keep the
 // per-image passes: 320 <- 416 channels, 5x5 at 40x40: 69 us an image, 71 by
 // phases)
+static int phase_rows(const ConvGeom &g) { return (g.F + PH_BK - 1) / PH_BK * PH_BK; }
 static bool dgrad_phases(const ConvGeom &g)
 {
     const long long own = ((long long)g.C * g.KS * g.KS + 127) / 128 * ((g.OH * g.OW + 127) / 128);
-    return own < 240 && g.S > 1 && g.S <= PH_MAX_S && g.S <= g.H && g.S <= g.W && !fc_geom(g);
+    // (the padded filter is addressed with 32-bit byte offsets)
+    return own < 240 && (double)phase_rows(g) * g.KS * g.KS * g.C < 536870911.0 && g.S > 1 && g.S <= PH_MAX_S && g.S <= g.H && g.S <= g.W && !fc_geom(g);
 }
 static PhaseTable phase_table(const ConvGeom &g)
 {
     PhaseTable t{};
+    t.fp = phase_rows(g);
+    t.dfp = make_fastdiv((unsigned)t.fp);
     int k = 0;
     for (int a = 0; a < g.S; ++a)
         for (int b = 0; b < g.S; ++b) {
@@ -3320,9 +3393,8 @@ static PhaseTable phase_table(const ConvGeom &g)
             p.w = (g.W - b + g.S - 1) / g.S;
             p.n = g.B * p.h * p.w;
             p.k0 = k;
-            p.nk = g.F * ta * tb;
+            p.nk = t.fp * ta * tb;
             p.tb = tb > 0 ? tb : 1;
-            p.dt = make_fastdiv((unsigned)(ta * tb > 0 ? ta * tb : 1));
             p.dtb = make_fastdiv((unsigned)p.tb);
             p.dhw = make_fastdiv((unsigned)(p.h * p.w));
             p.dw = make_fastdiv((unsigned)p.w);
@@ -3350,24 +3422,24 @@ static int dgrad_parts(const ConvGeom &g)
     const int bm = g.C <= 32 ? 32 : (g.C <= 64 ? 64 : 128), ph = g.S * g.S;
     const long long n0 = (long long)g.B * ((g.H + g.S - 1) / g.S) * ((g.W + g.S - 1) / g.S);
     const long long wgs = (g.C + bm - 1) / bm * ((n0 + 127) / 128) * ph;
-    const long long kt = (long long)g.F * g.KS * g.KS / ph / 16;
+    const long long kt = (long long)phase_rows(g) * g.KS * g.KS / ph / PH_BK;
     long long p = 512 / wgs;
     if (p > kt / 8) p = kt / 8;
     return p < 1 ? 1 : (p > 16 ? 16 : (int)p);
 }
 static size_t phase_filter_bytes(const ConvGeom &g)
 {
-    return ((size_t)g.F * g.C * g.KS * g.KS * sizeof(float) + 255) & ~(size_t)255;
+    return ((size_t)phase_rows(g) * g.C * g.KS * g.KS * sizeof(float) + 255) & ~(size_t)255;
 }
 // ws: the filter by phases, then the parts' sums where they fit
 static int dgrad_phases_launch(const ConvGeom &g, const float *dy, const float *w, float *dx,
                                void *ws, size_t ws_bytes, hipStream_t st)
 {
     const PhaseTable t = phase_table(g);
-    const int K = g.F * g.KS * g.KS, total = K * g.C;
+    const int K = t.fp * g.KS * g.KS, total = K * g.C;
     float *const wp = (float *)ws;
     hipLaunchKernelGGL(k_phase_filters, dim3((total + 255) / 256), dim3(256), 0, st, w, wp, g.C,
-                       g.KS, g.S, total, make_fastdiv((unsigned)g.C), t);
+                       g.F, g.KS, g.S, total, make_fastdiv((unsigned)g.C), t);
     int rc = check_launch();
     if (rc) return rc;
     const size_t n = (size_t)g.B * g.C * g.H * g.W, fb = phase_filter_bytes(g);
@@ -3499,7 +3571,7 @@ int ach_conv_bwd_data(const ach_conv_desc *d, const float *dy, const float *w, f
         return fwd_impl(dgrad_as_fwd(g), dy, wf, dx, part, ws_bytes - fb, st, Epi(), false, false);
     }
     if (!xy && dgrad_phases(g) &&
-        ws_bytes >= (size_t)g.F * g.C * g.KS * g.KS * sizeof(float))
+        ws_bytes >= (size_t)phase_rows(g) * g.C * g.KS * g.KS * sizeof(float))
         return dgrad_phases_launch(g, dy, w, dx, ws, ws_bytes, st);
     // Unequal strides, strides above PH_MAX_S or a workspace for one image's
     // columns only: the reference's per-image TN GEMM + col2im

@@ -235,6 +235,72 @@ def test_strided_input_gradient(gpu, shape):
         assert np.all(abs(dx.numpy() - ref) <= F * k * k * 2.0 ** -24 * mag)
 
 
+STRIDED = [
+    # (B, C, H, W, F, k, s, p): taps beyond dy's edge at some pixels
+    (2, 33, 8, 11, 70, 5, 2, 2),     # filters padded to k-tiles, ragged channels
+    (4, 32, 64, 64, 64, 5, 2, 2),    # nine taps of 64 filters
+    (2, 64, 28, 28, 96, 3, 2, 1),
+    (1, 12, 13, 13, 9, 5, 4, 3),
+]
+
+
+def run_strided(gpu, dy, w, shape):
+    B, Cc, H, W, F, k, s, p = shape
+    d = aetcnn.ConvDesc(B, Cc, H, W, F, k, s, p)
+    nb = gpu.ach_conv_bwd_data_workspace(C.byref(d))
+    ws, ddy, dw, dx = D(nb // 4 + 64), D.from_numpy(dy), D.from_numpy(w), D((B, Cc, H, W))
+    check(gpu.ach_conv_bwd_data(C.byref(d), ddy.ptr, dw.ptr, dx.ptr, ws.ptr, nb, None))
+    return dx.numpy().astype(np.float64)
+
+
+def strided_data(shape):
+    B, Cc, H, W, F, k, s, p = shape
+    rng = np.random.default_rng(sum(shape))
+    w = rng.standard_normal((F, Cc, k, k)).astype(np.float32)
+    oh, ow = (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+    return rng.standard_normal((B, F, oh, ow)).astype(np.float32), w
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("shape", STRIDED, ids=lambda s: "x".join(map(str, s)))
+def test_strided_input_gradient_non_finite(gpu, shape, value):
+    """A non-finite weight or delta reaches the pixels that its taps meet and
+    no other: a tap beyond dy's edge adds nothing (col2im adds no such term),
+    where a product with a padding zero would add a NaN."""
+    B, Cc, H, W, F, k, s, p = shape
+    for i, j in ((0, 0), (k - 1, k - 1), (k // 2, 0)):
+        dy, w = strided_data(shape)
+        w[F - 1, 1, i, j] = value
+        dy[0, 0, 0, 0] = dy[B - 1, 2, -1, -1] = value
+        got = run_strided(gpu, dy, w, shape)
+        with np.errstate(invalid="ignore"):
+            ref = refs64.dgrad_ref(dy, w, (B, Cc, H, W), s, p)
+        assert np.isfinite(ref).any() and not np.isfinite(ref).all()
+        assert np.array_equal(np.isnan(got), np.isnan(ref))
+        assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+        fin = np.isfinite(ref)
+        assert np.all(abs(got[fin] - ref[fin]) <= 1e-5 * abs(ref[fin]).max())
+
+
+@pytest.mark.parametrize("shape", STRIDED[1:3], ids=lambda s: "x".join(map(str, s)))
+def test_strided_input_gradient_error(gpu, shape):
+    """Each tap's sum over the filters stands by itself.  A rounding of a sum
+    is uniform within half a unit in the last place, at most 2^-24 / sqrt(3)
+    of it; a chain of F products rounds at most F times while the sum grows
+    evenly, so the squares add to F/2 of the last one's, and the taps'
+    additions to another half of their number:
+    relative rms error <= 2^-24 sqrt((F + taps) / 2 / 3).  (One chain over
+    filters and taps is at 1.3 to 2.5 times the error of these sums.)"""
+    B, Cc, H, W, F, k, s, p = shape
+    dy, w = strided_data(shape)
+    ref = refs64.dgrad_ref(dy, w, (B, Cc, H, W), s, p)
+    err = np.linalg.norm(run_strided(gpu, dy, w, shape) - ref) / np.linalg.norm(ref)
+    taps = (k / s) ** 2
+    limit = 2.0 ** -24 * ((F + taps) / 6) ** 0.5
+    print(f"{shape}: {err:.2e}, bound {limit:.2e}")
+    assert err <= limit
+
+
 @pytest.mark.parametrize("B,K,F", [
     (33, 128, 128),      # two row fragments, one of them a single row; one tile
     (64, 300, 130),      # K not a multiple of 8, ragged features
