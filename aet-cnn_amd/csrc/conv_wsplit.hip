@@ -249,21 +249,31 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
 #pragma unroll 1
             for (int s = s0; s < s1; ++s) {
                 const int un = fdiv(s, p.dh), iy = s - un * p.H, im = fdiv(un, p.dnu);
-                const int oy = iy - q / KS + P, cb = (un - im * p.nu) * p.cols;
-                if (oy < 0 || oy >= p.H) continue;
+                const int cb = (un - im * p.nu) * p.cols, oy0 = iy - q / KS + P;
+                // the dy row that this tap row meets beyond x's first or last
+                // row (products with padding zeros, which no step forms) goes
+                // with that row of x
+                const int edge = iy == 0 && q / KS < P             ? P - 1 - q / KS
+                                 : iy == p.H - 1 && q / KS > P     ? p.H - q / KS + P
+                                                                   : -1;
 #pragma unroll 1
-                for (int e = 0; e < 16; ++e) {
-                    const int b = p.pair ? 2 * im + (e >> 3) : im;
-                    const int ox = cb + (p.pair ? e & 7 : e), ix = ox + q % KS - P;
-                    if (b >= p.B || ox >= p.W) continue;
-                    float xv = 0.f;
-                    if (c < p.C && ix >= 0 && ix < p.W)
-                        xv = p.x[(((size_t)b * p.C + c) * p.H + iy) * p.W + ix];
+                for (int t = 0; t < 2; ++t) {
+                    const int oy = t ? edge : oy0;
+                    if (oy < 0 || oy >= p.H) continue;
+#pragma unroll 1
+                    for (int e = 0; e < 16; ++e) {
+                        const int b = p.pair ? 2 * im + (e >> 3) : im;
+                        const int ox = cb + (p.pair ? e & 7 : e), ix = ox + q % KS - P;
+                        if (b >= p.B || ox >= p.W) continue;
+                        float xv = 0.f;
+                        if (!t && c < p.C && ix >= 0 && ix < p.W)
+                            xv = p.x[(((size_t)b * p.C + c) * p.H + iy) * p.W + ix];
 #pragma unroll
-                    for (int g = 0; g < 16; ++g) {
-                        const int fr = f + 8 * (g >> 2) + (g & 3);
-                        if (fr < p.F)
-                            a[g] += p.dy[(((size_t)b * p.F + fr) * p.H + oy) * p.W + ox] * xv;
+                        for (int g = 0; g < 16; ++g) {
+                            const int fr = f + 8 * (g >> 2) + (g & 3);
+                            if (fr < p.F)
+                                a[g] += p.dy[(((size_t)b * p.F + fr) * p.H + oy) * p.W + ox] * xv;
+                        }
                     }
                 }
             }

@@ -202,6 +202,30 @@ def test_weight_gradient_non_finite(gpu, value):
                 assert np.array_equal(np.sign(got[:, 70, i, j]), np.sign(dy[5, :, 4 - i, 4 - j]))
 
 
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("shape", [WGRAD[0], WGRAD[2]], ids=lambda s: "x".join(map(str, s)))
+def test_weight_gradient_non_finite_delta(gpu, shape, value):
+    """A non-finite delta meets the padding around the input as zeros, as in
+    im2col: every tap that looks beyond an edge from its position is NaN."""
+    B, Cc, H, W, F = shape
+    rng = np.random.default_rng(7)
+    x = rng.standard_normal((B, Cc, H, W)).astype(np.float32)
+    dy = rng.standard_normal((B, F, H, W)).astype(np.float32)
+    at = {0: (0, 0, 0), 40: (B - 1, H - 1, W - 1), 70: (1, 0, W // 2), 131: (B // 2, H - 1, 1),
+          200: (2, H // 2, W - 1), 255: (3, H // 2, 2)}  # filter: image, row, column
+    for f, (b, i, j) in at.items():
+        dy[b, f, i, j] = value
+    got = run_wgrad(gpu, x, dy, np.zeros((F, Cc, 3, 3), np.float32))
+    with np.errstate(invalid="ignore"):
+        ref = refs64.wgrad_ref(x, dy[:, list(at)], 3, 1, 1)
+    some = got[list(at)]
+    if np.isinf(value):  # taps within the image are infinite, those beyond it NaN
+        assert not np.isnan(ref[5]).any() and np.isnan(ref[0]).sum() == 5 * Cc
+    assert np.array_equal(np.isnan(some), np.isnan(ref))
+    assert np.array_equal(some[np.isinf(ref)], ref[np.isinf(ref)])
+    assert np.isfinite(np.delete(got, list(at), 0)).all()
+
+
 @pytest.mark.parametrize("shape", [
     # (B, C, H, W, F, k, s, p): input gradients by phases
     (3, 48, 9, 7, 20, 3, 2, 1),
