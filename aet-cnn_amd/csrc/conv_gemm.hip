@@ -3414,9 +3414,12 @@ static int dgrad_phases_bm(const ConvGeom &g, const PhaseTable &t, const float *
     DgradPhase<BM, false> p{dy, wp, dx, g, g.C, K, parts, t};
     return launch_gemm(p, g.C, nmax, t.n * parts, st);
 }
-// K parts of every phase: enough for two workgroups per CU, eight k-tiles each
+// K parts of every phase: enough for two workgroups per CU, three k-tiles each
 // on average (320 <- 416 channels, 5x5 stride 2 at 40x40, batch 3: 120
-// workgroups of 234 k-tiles took 385 us)
+// workgroups of 234 k-tiles took 385 us).  With eight k-tiles a single image
+// ran longer than its own GEMM and col2im: 64 <- 96 channels 3x3 at 14x14 22.2
+// us by image, 27.2 with eight, 15.8 with three; 400 <- 300 at 40x40 52.2,
+// 59.4, 47.8.
 static int dgrad_parts(const ConvGeom &g)
 {
     const int bm = g.C <= 32 ? 32 : (g.C <= 64 ? 64 : 128), ph = g.S * g.S;
@@ -3424,7 +3427,7 @@ static int dgrad_parts(const ConvGeom &g)
     const long long wgs = (g.C + bm - 1) / bm * ((n0 + 127) / 128) * ph;
     const long long kt = (long long)phase_rows(g) * g.KS * g.KS / ph / PH_BK;
     long long p = 512 / wgs;
-    if (p > kt / 8) p = kt / 8;
+    if (p > kt / 3) p = kt / 3;
     return p < 1 ? 1 : (p > 16 ? 16 : (int)p);
 }
 static size_t phase_filter_bytes(const ConvGeom &g)
