@@ -13,9 +13,13 @@
 //
 // Non-finite values: an infinity (or a finite value above 2^103, which the
 // operands' scale of 2^24 takes to one) leaves non-finite residuals, so the
-// tile's sums come out non-finite; a wave
-// that finds a non-finite sum recomputes its tile in plain fp32, which gives
-// the infinities and NaNs of fp32 arithmetic.
+// tile's sums come out non-finite; a wave that finds a non-finite sum
+// computes its tile again on the fp32 instructions, straight from memory,
+// which gives the infinities and NaNs of fp32 arithmetic (and, a channel
+// chunk's sums standing by themselves, no more error than the fp32 kernels:
+// 2.2e-7 against 6.0e-7 for 128 -> 128 @ 32x32 at 1e35).  With NaNs
+// everywhere that layer takes 560 us, 172 without and 310 on the fp32 kernel;
+// one NaN in the batch takes it to 240.
 //
 // The workgroup: four waves of 32 filters x 128 positions (2 x 64 or 1 x 32
 // for 33-64 or up to 32 filters).  A chunk of 16 input channels of the tile's
@@ -276,34 +280,55 @@ __global__ void __launch_bounds__(64 * WM * WN * KG, 2) k_conv_split(SplitFwd p)
             hi[f][r] += lo[f][r];
             bad |= !(fabsf(hi[f][r]) <= 3.402823466e38f);
         }
-    if (__ballot(bad)) {  // rare: recompute this wave's tile in fp32
-        const int mb = m0 + wm * 32 + 4 * half;
+    if (__ballot(bad)) {  // this wave's tile again on the fp32 instructions
+        int xo[NF], oy[NF], ox[NF];
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
             const int n = n0 + (wn * NF + f) * 32 + l32;
-            const int b = fdiv(n, p.dohw), pos = n - b * OHW;
-            const int oh = fdiv(pos, p.dow), ow = pos - oh * p.OW;
-            v16f s;
+            const int b = fdiv(n, p.dohw), pos = n - b * OHW, oh = fdiv(pos, p.dow);
+            oy[f] = n < p.N ? oh - p.P : p.H;  // (past the end: no row is inside)
+            ox[f] = pos - oh * p.OW - p.P;
+            xo[f] = b * p.C * HW + oy[f] * p.W + ox[f];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = 0.f;
-            const int cend = min(p.C, ch1 * SP_CH);
-#pragma unroll 1
-            for (int c = ch0 * SP_CH; c < cend; ++c)
-#pragma unroll 1
-                for (int tap = 0; tap < T; ++tap) {
-                    const int ih = oh + tap / KS - p.P, iw = ow + tap % KS - p.P;
-                    float xv = 0.f;
-                    if (n < p.N && ih >= 0 && ih < p.H && iw >= 0 && iw < p.W)
-                        xv = p.x[((size_t)b * p.C + c) * HW + ih * p.W + iw];
-                    const float *w = p.wt + (size_t)(c * T + tap) * p.M;
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int mm = mb + 8 * (r >> 2) + (r & 3);
-                        if (mm < p.M) s[r] += w[mm] * xv;
-                    }
-                }
-            hi[f] = s;
+            for (int r = 0; r < 16; ++r) hi[f][r] = lo[f][r] = 0.f;
         }
+        const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, xbytes), rw = make_rsrc(p.wt, wbytes);
+        const int cend = min(p.C, ch1 * SP_CH);
+#pragma unroll 1
+        for (int c0 = ch0 * SP_CH; c0 < cend; c0 += 2) {  // lane half h: channel c0 + h
+            const int c = c0 + half;
+            // a chunk's sums stand by themselves: one chain over all channels
+            // had up to twice the error of the fp32 kernels' K parts
+            if (c0 % SP_CH == 0) {
+#pragma unroll
+                for (int f = 0; f < NF; ++f) {
+                    hi[f] += lo[f];
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) lo[f][r] = 0.f;
+                }
+            }
+#pragma unroll 1
+            for (int ki = 0; ki < KS; ++ki) {
+                float av[KS], bv[NF][KS];
+#pragma unroll
+                for (int kj = 0; kj < KS; ++kj) {
+                    av[kj] = bload(rw, boff((c < cend) & (m < p.M),
+                                            (c * T + ki * KS + kj) * p.M + m));
+#pragma unroll
+                    for (int f = 0; f < NF; ++f)
+                        bv[f][kj] = bload(rx, boff((c < cend) & ((unsigned)(oy[f] + ki) < (unsigned)p.H) &
+                                                       ((unsigned)(ox[f] + kj) < (unsigned)p.W),
+                                                   xo[f] + c * HW + ki * p.W + kj));
+                }
+#pragma unroll
+                for (int kj = 0; kj < KS; ++kj)
+#pragma unroll
+                    for (int f = 0; f < NF; ++f)
+                        lo[f] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[kj], bv[f][kj], lo[f], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int f = 0; f < NF; ++f) hi[f] += lo[f];
     } else {
 #pragma unroll
         for (int f = 0; f < NF; ++f)

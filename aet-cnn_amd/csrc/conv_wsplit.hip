@@ -27,6 +27,11 @@
 // reduction, batch 128, fp32 kernel before -> now: 128 -> 128 @ 32x32 293 ->
 // 189 us (205 TFLOP/s), 512 -> 512 @ 8x8 295 -> 187, 384 -> 384 @ 13x13 477
 // -> 325 (rows of 13 of 16 positions); batch 32, 512 -> 512 @ 8x8 88 -> 69.
+// Non-finite sums are computed again as in conv_split.hip: with NaNs
+// everywhere the first of these takes 920 us (310 on the fp32 kernel).  What
+// the recomputation keeps in registers is counted beside the loop's: written
+// with indexed sums it made the kernel spill 82 registers after the loop
+// (188 us instead of 183, 62.9 MB written a launch instead of 37.7).
 // Partial sums laid out [tap][f][c], 32 channels a line: stored as dw is
 // ([f][c][tap], 36 bytes between lanes) the first of these took 237 us.
 #include "conv_wsplit.hpp"
@@ -240,50 +245,61 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
 #pragma unroll
         for (int e = 0; e < 16; ++e) bad |= !(fabsf(acc[q / KS][q % KS][e]) <= 3.402823466e38f);
     const int c = c0 + wc * 32 + l32, f = m0 + wf * 32 + 4 * half;
-    if (__ballot(bad)) {  // rare: recompute this wave's tiles in fp32
-#pragma unroll
-        for (int q = 0; q < T; ++q) {
-            v16f a;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) a[e] = 0.f;
-#pragma unroll 1
-            for (int s = s0; s < s1; ++s) {
-                const int un = fdiv(s, p.dh), iy = s - un * p.H, im = fdiv(un, p.dnu);
-                const int cb = (un - im * p.nu) * p.cols, oy0 = iy - q / KS + P;
-                // the dy row that this tap row meets beyond x's first or last
-                // row (products with padding zeros, which no step forms) goes
-                // with that row of x
-                const int edge = iy == 0 && q / KS < P             ? P - 1 - q / KS
-                                 : iy == p.H - 1 && q / KS > P     ? p.H - q / KS + P
-                                                                   : -1;
-#pragma unroll 1
-                for (int t = 0; t < 2; ++t) {
-                    const int oy = t ? edge : oy0;
-                    if (oy < 0 || oy >= p.H) continue;
-#pragma unroll 1
-                    for (int e = 0; e < 16; ++e) {
-                        const int b = p.pair ? 2 * im + (e >> 3) : im;
-                        const int ox = cb + (p.pair ? e & 7 : e), ix = ox + q % KS - P;
-                        if (b >= p.B || ox >= p.W) continue;
-                        float xv = 0.f;
-                        if (!t && c < p.C && ix >= 0 && ix < p.W)
-                            xv = p.x[(((size_t)b * p.C + c) * p.H + iy) * p.W + ix];
-#pragma unroll
-                        for (int g = 0; g < 16; ++g) {
-                            const int fr = f + 8 * (g >> 2) + (g & 3);
-                            if (fr < p.F)
-                                a[g] += p.dy[(((size_t)b * p.F + fr) * p.H + oy) * p.W + ox] * xv;
-                        }
-                    }
-                }
-            }
-            acc[q / KS][q % KS] = a;
-        }
-    } else {
+    float down = kSumDown;
+    if (__ballot(bad)) {  // this wave's tiles again on the fp32 instructions
+        down = 1.f;
 #pragma unroll
         for (int q = 0; q < T; ++q)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[q / KS][q % KS][e] *= kSumDown;
+            for (int e = 0; e < 16; ++e) acc[q / KS][q % KS][e] = 0.f;
+        const int fr = m0 + wf * 32 + l32;
+        const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, (unsigned)((size_t)p.B * p.C * HW * 4));
+        const __amdgpu_buffer_rsrc_t rd = make_rsrc(p.dy, (unsigned)((size_t)p.B * p.F * HW * 4));
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+#pragma unroll 1
+            for (int s = s0; s < s1; ++s) {  // lane half h: segment h
+                const int un = fdiv(s, p.dh), iy = s - un * p.H, q = fdiv(un, p.dnu);
+                const int cb = (un - q * p.nu) * p.cols, b = (q << ps) + (ps ? half : 0);
+                const int ox0 = cb + (ps ? 0 : half * 8);
+                const bool okf = (fr < p.F) & (b < p.B), okc = (c < p.C) & (b < p.B);
+                const int xrow = (b * p.C + c) * HW + iy * p.W, drow = (b * p.F + fr) * HW;
+                // t = 1: the dy row that this tap row meets beyond x's first
+                // or last row, with that row of x (products with padding
+                // zeros, which no step forms)
+                const int edge = (iy == 0 && i < P) || (iy == p.H - 1 && i > P);
+#pragma unroll 1
+                for (int t = 0; t <= edge; ++t) {
+                    const int oy = t ? iy : iy - i + P;
+                    if (oy < 0 || oy >= p.H) continue;
+                    float dv[8], xv[10];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        dv[e] = bload(rd, boff(okf & (ox0 + e < p.W), drow + oy * p.W + ox0 + e));
+#pragma unroll
+                    for (int e = 0; e < 10; ++e)
+                        xv[e] = bload(rx, boff(okc & !t & ((unsigned)(ox0 + e - P) < (unsigned)p.W),
+                                               xrow + ox0 + e - P));
+                    // a row's sums stand by themselves, as one chain over the
+                    // slice had more error than the fp32 kernel's shorter ones
+                    v16f sum[KS];
+#pragma unroll
+                    for (int j = 0; j < KS; ++j)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) sum[j][r] = 0.f;
+                    // (a position past the row's end meets no x: its zero
+                    // delta must not meet an infinite one)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+#pragma unroll
+                        for (int j = 0; j < KS; ++j)
+                            sum[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                                dv[e], ox0 + e < p.W ? xv[e + j] : 0.f, sum[j], 0, 0, 0);
+#pragma unroll
+                    for (int j = 0; j < KS; ++j) acc[i][j] += sum[j];
+                }
+            }
+        }
     }
     // the groups exchange tiles in rounds of QR taps: group q & 1 stores tap q
     constexpr int QR = 4;
@@ -294,7 +310,7 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
 #pragma unroll
         for (int q = q0; q < (q0 + QR < T ? q0 + QR : T); ++q)
             if ((q & 1) != grp) {
-                const v16f &t = acc[q / KS][q % KS];
+                const v16f t = acc[q / KS][q % KS] * down;
 #pragma unroll
                 for (int r4 = 0; r4 < 4; ++r4)
                     xs[((q - q0) * 4 + r4) * NT + tid] =
@@ -304,7 +320,7 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
 #pragma unroll
         for (int q = q0; q < (q0 + QR < T ? q0 + QR : T); ++q)
             if ((q & 1) == grp) {
-                const v16f &t = acc[q / KS][q % KS];
+                const v16f t = acc[q / KS][q % KS] * down;
                 const int ld = p.C;
                 float *base = p.part + (((size_t)z * T + q) * p.F + f) * ld + c;
 #pragma unroll

@@ -143,7 +143,7 @@ __global__ void __launch_bounds__(256, 2) k_fc_split(FcSplit p)
     }
     // the weight gradient's prior values, all loads in flight at once
     float old[MODE == 2 ? MT : 1][NT][16];
-    if constexpr (MODE == 2) {
+    auto load_old = [&](auto each) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -153,11 +153,13 @@ __global__ void __launch_bounds__(256, 2) k_fc_split(FcSplit p)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
                     const int dr = 8 * (e >> 2) + (e & 3);
-                    hi[i][j][e] += lo[i][j][e];
+                    each(i, j, e);
                     old[i][j][e] = c < p.N && r + dr < p.R ? base[(size_t)dr * p.N] : 0.f;
                 }
             }
-    }
+    };
+    if constexpr (MODE == 2)
+        load_old([&](int i, int j, int e) { hi[i][j][e] += lo[i][j][e]; });
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < MT; ++i)
@@ -168,35 +170,59 @@ __global__ void __launch_bounds__(256, 2) k_fc_split(FcSplit p)
                 if constexpr (MODE != 2) hi[i][j][e] += lo[i][j][e];
                 bad |= !(fabsf(hi[i][j][e]) <= 3.402823466e38f);
             }
-    if (__ballot(bad)) {  // rare: recompute this wave's tiles in fp32
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                const int r = m0 + (wm * MT + i) * 32 + 4 * half, c = n0 + (wn * NT + j) * 32 + l32;
-                v16f s;
-#pragma unroll
-                for (int e = 0; e < 16; ++e) s[e] = 0.f;
-#pragma unroll 1
-                for (int k = k0; k < k1; ++k) {
-                    float bv = 0.f;
-                    if (c < p.N) bv = BKM ? p.b[(size_t)k * p.N + c] : p.b[(size_t)c * p.K + k];
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        const int rr = r + 8 * (e >> 2) + (e & 3);
-                        if (rr < p.R)
-                            s[e] += (AK ? p.a[(size_t)k * p.R + rr] : p.a[(size_t)rr * p.K + k]) * bv;
-                    }
-                }
-                hi[i][j] = s;
-            }
-    } else {
+    float down = kSumDown;
+    if (__ballot(bad)) {  // this wave's tiles again on the fp32 instructions
+        down = 1.f;
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int j = 0; j < NT; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) hi[i][j][e] *= kSumDown;
+                for (int e = 0; e < 16; ++e) hi[i][j][e] = lo[i][j][e] = 0.f;
+        auto at = [&](bool km, int row, int total, int k) {
+            return boff((row < total) & (k < k1), km ? k * total + row : row * p.K + k);
+        };
+        // (a chunk's sums stand by themselves: one chain had up to 1.4 times
+        // the error of the fp32 kernels' K parts)
+        constexpr int U = 4;
+#pragma unroll 1
+        for (int kc = k0; kc < k1; kc += 2 * U) {  // lane half h: k = kc + 2u + h
+            if (((kc - k0) & (FP_K - 1)) == 0) {
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) {
+                        hi[i][j] += lo[i][j];
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) lo[i][j][e] = 0.f;
+                    }
+            }
+            float av[U][MT], bv[U][NT];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int k = kc + 2 * u + half;
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+                    av[u][i] = bload(ra, at(AK, m0 + (wm * MT + i) * 32 + l32, p.R, k));
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    bv[u][j] = bload(rb, at(BKM, n0 + (wn * NT + j) * 32 + l32, p.N, k));
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+                        lo[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[u][i], bv[u][j], lo[i][j],
+                                                                        0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) hi[i][j] += lo[i][j];
+        // (read again: kept over the recomputation they would not fit)
+        if constexpr (MODE == 2) load_old([](int, int, int) {});
     }
 #pragma unroll
     for (int i = 0; i < MT; ++i)
@@ -218,7 +244,7 @@ __global__ void __launch_bounds__(256, 2) k_fc_split(FcSplit p)
                 for (int e = 0; e < 16; ++e) {
                     const int dr = 8 * (e >> 2) + (e & 3);
                     if (r + dr >= p.R) continue;
-                    float u = old[i][j][e] + hi[i][j][e];
+                    float u = old[i][j][e] + hi[i][j][e] * down;
                     if (wb) {
                         sgd_step(wv[e], u, p.sg.dc, p.sg.lc, p.sg.mom);
                         wb[(size_t)dr * p.N] = wv[e];
@@ -231,7 +257,7 @@ __global__ void __launch_bounds__(256, 2) k_fc_split(FcSplit p)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
                     const int dr = 8 * (e >> 2) + (e & 3);
-                    float v = hi[i][j][e];
+                    float v = hi[i][j][e] * down;
                     if constexpr (MODE == 1) v = p.e.apply(v, c);
                     if (r + dr < p.R) base[(size_t)dr * p.N] = v;
                 }

@@ -226,6 +226,96 @@ def test_weight_gradient_non_finite_delta(gpu, shape, value):
     assert np.isfinite(np.delete(got, list(at), 0)).all()
 
 
+def rel_rms(a, ref):
+    return float(np.linalg.norm(a - ref) / np.linalg.norm(ref))
+
+
+def test_large_values_error(gpu):
+    """Values above 2^103 take the fp32 instructions, in blocks of L products
+    whose sums are added one by one.  With roundings uniform within half a
+    unit and sums that grow evenly: relative rms error <=
+    2^-24 sqrt((L + blocks) / 6)."""
+    rng = np.random.default_rng(21)
+
+    def draw(scale, *shape):
+        return (rng.standard_normal(shape) * scale).astype(np.float32)
+
+    def bound(block, blocks):
+        return 2.0 ** -24 * ((block + blocks) / 6) ** 0.5
+
+    B, Cc, H, W, F = 8, 128, 16, 16, 128
+    x, w = draw(1e35, B, Cc, H, W), draw(1e-36, F, Cc, 3, 3)
+    d = aetcnn.ConvDesc(B, Cc, H, W, F, 3, 1, 1)
+    nb = gpu.ach_conv_fwd_workspace(C.byref(d))
+    ws, dx, dw, y = D(nb // 4 + 64), D.from_numpy(x), D.from_numpy(w), D((B, F, H, W))
+    check(gpu.ach_conv_fwd(C.byref(d), dx.ptr, dw.ptr, y.ptr, ws.ptr, nb, None))
+    e = rel_rms(y.numpy(), refs64.conv_ref(x, w, 1, 1))
+    print(f"forward {e:.2e}, bound {bound(9 * 16, Cc // 16):.2e}")
+    assert e <= bound(9 * 16, Cc // 16)
+    # 832 row steps in at least ten slices
+    B, Cc, H, W, F = WGRAD[2]
+    x, dy = draw(1e35, B, Cc, H, W), draw(1e-36, B, F, H, W)
+    got = run_wgrad(gpu, x, dy, np.zeros((F, Cc, 3, 3), np.float32)).astype(np.float64)
+    e = rel_rms(got, wgrad_ref(x.astype(np.float64), dy.astype(np.float64)))
+    print(f"weight gradient {e:.2e}, bound {bound(16, 84):.2e}")
+    assert e <= bound(16, 84)
+    B, K, F = 128, 2900, 2900
+    x, w, dy = draw(1e35, B, K), draw(1e-36, F, K), draw(1e-36, B, F)
+    d = aetcnn.ConvDesc(B, K, 1, 1, F, 1, 1, 0)
+    nb = max(gpu.ach_conv_fwd_workspace(C.byref(d)), gpu.ach_conv_bwd_filter_workspace(C.byref(d)))
+    ws, dx, dw, ddy, y, g = D(nb // 4 + 64), *map(D.from_numpy, (x, w, dy)), D((B, F)), D((F, K))
+    g.zero()
+    check(gpu.ach_conv_fwd(C.byref(d), dx.ptr, dw.ptr, y.ptr, ws.ptr, nb, None))
+    check(gpu.ach_conv_bwd_filter(C.byref(d), dx.ptr, ddy.ptr, g.ptr, ws.ptr, nb, None))
+    x, w, dy = (a.astype(np.float64) for a in (x, w, dy))
+    for name, a, ref, n in (("fc forward", y, x @ w.T, K), ("fc weight gradient", g, dy.T @ x, B)):
+        e = rel_rms(a.numpy(), ref)
+        print(f"{name} {e:.2e}, bound {bound(32, n / 32):.2e}")
+        assert e <= bound(32, n / 32)
+
+
+@pytest.mark.parametrize("dims", [(128, 128, 32, 32, 128, 3, 1), (128, 96, 27, 27, 256, 5, 2),
+                                  (128, 4096, 1, 1, 4096, 1, 0)], ids=lambda s: "x".join(map(str, s)))
+def test_time_of_non_finite_calls(gpu, dims):
+    """A diverged network's calls stay within ten times a finite call's time
+    (every tile is then computed twice, once on the slower instructions)."""
+    B, Cc, H, W, F, k, p = dims
+    rng = np.random.default_rng(2)
+    d = aetcnn.ConvDesc(B, Cc, H, W, F, k, 1, p)
+    r = C.byref(d)
+    nb = max(gpu.ach_conv_fwd_workspace(r), gpu.ach_conv_bwd_data_workspace(r),
+             gpu.ach_conv_bwd_filter_workspace(r))
+    ws, w = D(nb // 4 + 64), D.from_numpy(rng.standard_normal((F, Cc, k, k)).astype(np.float32))
+    finite = D.from_numpy(rng.standard_normal(B * max(Cc, F) * H * W).astype(np.float32))
+    nans = D.from_numpy(np.full(B * max(Cc, F) * H * W, np.nan, np.float32))
+    out = D(max(B * max(Cc, F) * H * W, F * Cc * k * k))
+    ev = [C.c_void_p() for _ in range(2)]
+    for e in ev:
+        check(gpu.ach_event_create(C.byref(e)))
+
+    def time(call):
+        ms = C.c_float()
+        call()
+        check(gpu.ach_event_record(ev[0], None))
+        call()
+        check(gpu.ach_event_record(ev[1], None))
+        check(gpu.ach_event_sync(ev[1]))
+        check(gpu.ach_event_elapsed_ms(ev[0], ev[1], C.byref(ms)))
+        return ms.value
+
+    for name, call in (
+            ("forward", lambda a: gpu.ach_conv_fwd(r, a.ptr, w.ptr, out.ptr, ws.ptr, nb, None)),
+            ("input gradient",
+             lambda a: gpu.ach_conv_bwd_data(r, a.ptr, w.ptr, out.ptr, ws.ptr, nb, None)),
+            ("weight gradient",
+             lambda a: gpu.ach_conv_bwd_filter(r, a.ptr, a.ptr, out.ptr, ws.ptr, nb, None))):
+        t = [time(lambda: check(call(a))) for a in (finite, nans)]
+        print(f"{name}: {t[0] * 1e3:.0f} us, NaNs {t[1] * 1e3:.0f} us")
+        assert t[1] <= 10 * t[0], name
+    for e in ev:
+        check(gpu.ach_event_destroy(e))
+
+
 @pytest.mark.parametrize("shape", [
     # (B, C, H, W, F, k, s, p): input gradients by phases
     (3, 48, 9, 7, 20, 3, 2, 1),
