@@ -1,6 +1,6 @@
-// Weight gradient of stride-1 convolutions that keep their size (k odd,
-// pad (k-1)/2): dW[f][c][ki][kj] = sum over images and positions of
-// dy[f][oy][ox] * x[c][oy+ki-P][ox+kj-P], on the bf16 matrix cores with
+// Weight gradient of 3x3 stride-1 convolutions with padding 1:
+// dW[f][c][ki][kj] = sum over images and positions of
+// dy[f][oy][ox] * x[c][oy+ki-1][ox+kj-1], on the bf16 matrix cores with
 // three exact bf16 pieces per float (the arithmetic of conv_split.hip).
 //
 // The contraction runs over positions, which are contiguous in both tensors,
@@ -9,10 +9,10 @@
 // step is one input row y of a unit: 16 positions as two segments of 8,
 // either adjacent columns of one image or, when the row has an odd number of
 // segments, the same segment of two images.  At a step a wave reads x's row
-// once, forms its k shifted versions in registers (a segment keeps its two
-// neighbours on each side beside it) and multiplies them with the dy rows
-// y-ki+P of a ring in LDS: one x row and one dy row are split and staged per
-// step for k*k taps of MFMAs.  Rows of consecutive units follow each other
+// once, forms its three shifted versions in registers (a segment keeps its
+// neighbour on each side beside it) and multiplies them with the dy rows
+// y-ki+1 of a ring in LDS: one x row and one dy row are split and staged per
+// step for nine taps of MFMAs.  Rows of consecutive units follow each other
 // in the ring, so a slice is any range of steps.
 //
 // A workgroup is 64 filters x 64 channels x 9 taps: two groups of four waves
@@ -59,7 +59,7 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
     constexpr int KS = 3, P = 1, NT = 256, T = KS * KS;
     constexpr int R = 64;                      // rows of dy (f) and of x (c) per workgroup
     constexpr int ROWB = 6 * R * 16;           // bytes of a staged row: [piece][seg][r] x 16
-    constexpr int NBB = 12 * R * 4;            // its neighbour pairs: [piece][seg][side][r] x 4
+    constexpr int NBB = 6 * R * 4;             // its neighbours: [piece][seg][r] x (right, left)
     constexpr int NR = KS + 1;                 // dy rows in the ring
     constexpr int GB = (NR + 1) * ROWB + 2 * (ROWB + NBB) + NBB;
     extern __shared__ __align__(16) char smem[];
@@ -87,8 +87,8 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
     const int HW = p.H * p.W;
 
     // Staging: waves 0 and 1 take 32 rows of dy each, 2 and 3 of x; a lane one
-    // segment (8 positions) of one row, and for x the two positions on each
-    // side of it.  A wave's role is a matter of operands, not of branches.
+    // segment (8 positions) of one row, and for x the position on each side
+    // of it.  A wave's role is a matter of operands, not of branches.
     const bool isx = wave >= 2;
     const int trow = (wave & 1) * 32 + (lane >> 1), seg = lane & 1;
     const int nrow = isx ? p.C : p.F, row = (isx ? c0 : m0) + trow;
@@ -105,7 +105,7 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
     const int ps = p.pair ? 1 : 0, segc = ps ? 0 : seg * 8, segb = ps ? seg : 0;
     const int lanebase = (row + segb * nrow) * HW + segc;
     char *const st0 = dyb + (trow + seg * R) * 16;
-    char *const st1 = dyb + (seg * 2 * R + trow) * 4;
+    char *const st1 = dyb + (seg * R + trow) * 4;
     auto load = [&](int s, float *r) {
         const int ds = s + lead, dc = max(ds, 0);
         const int u = fdiv(dc, p.dh), y = dc - u * p.H, q = fdiv(u, p.dnu);
@@ -124,10 +124,8 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
             for (int j = 0; j < 8; ++j) r[j] = bload(rs, (ok & (left > j)) ? base + 4 * j : (int)kOOB);
         }
         // the neighbours (a dy row has none: out-of-range offsets)
-        r[8] = bload(rs, ((ok & (col > 0) & (left > -2)) ? base - 8 : (int)kOOB) | side);
+        r[8] = bload(rs, ((ok & (left > 8)) ? base + 32 : (int)kOOB) | side);
         r[9] = bload(rs, ((ok & (col > 0) & (left > -1)) ? base - 4 : (int)kOOB) | side);
-        r[10] = bload(rs, ((ok & (left > 8)) ? base + 32 : (int)kOOB) | side);
-        r[11] = bload(rs, ((ok & (left > 9)) ? base + 36 : (int)kOOB) | side);
     };
     auto store = [&](int s, const float *r) {
         v4u pc[3];
@@ -137,16 +135,13 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
         unsigned *const nb = reinterpret_cast<unsigned *>(st1 + nb0 + slot * nbb);
 #pragma unroll
         for (int q = 0; q < 3; ++q) *reinterpret_cast<v4u *>(dst + q * 2 * R * 16) = pc[q];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const float a = r[8 + 2 * i] * kPieceUp, b = r[9 + 2 * i] * kPieceUp;
-            const unsigned h = pk_bf16(a, b);
-            const float ra = a - bf_lo(h), rb = b - bf_hi(h);
-            const unsigned m = pk_bf16(ra, rb);
-            nb[i * R] = h;
-            nb[4 * R + i * R] = m;
-            nb[8 * R + i * R] = pk_bf16(ra - bf_lo(m), rb - bf_hi(m));
-        }
+        const float a = r[8] * kPieceUp, b = r[9] * kPieceUp;
+        const unsigned h = pk_bf16(a, b);
+        const float ra = a - bf_lo(h), rb = b - bf_hi(h);
+        const unsigned m = pk_bf16(ra, rb);
+        nb[0] = h;
+        nb[2 * R] = m;
+        nb[4 * R] = pk_bf16(ra - bf_lo(m), rb - bf_hi(m));
     };
 
     v16f acc[KS][KS];
@@ -160,9 +155,9 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
     for (int i = tid * 16; i < ROWB; i += NT * 16) *reinterpret_cast<v4u *>(zero + i) = v4u{0, 0, 0, 0};
     // steps s0-2 and s0-1 bring the ring's first dy rows (their x rows go to
     // slots that later steps overwrite)
-    float r[12];
+    float r[10];
     {
-        float r0[12], r1[12], r2[12];
+        float r0[10], r1[10], r2[10];
         load(s0 - 2, r0);
         load(s0 - 1, r1);
         load(s0, r2);
@@ -179,14 +174,11 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
     for (int s = s0; s < s0 + p.spw; ++s) {
         const char *const xr = xb + (s & 1) * (ROWB + NBB);
         v4u u[3], a[2][3];
-        unsigned nl[3], nr[3];
+        unsigned nb[3];
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
             u[q] = *reinterpret_cast<const v4u *>(xr + frag + (q * 2 * R + wc * 32) * 16);
-            const unsigned *nb = reinterpret_cast<const unsigned *>(xr + ROWB) +
-                                 (q * 2 + half) * 2 * R + wc * 32 + l32;
-            nl[q] = nb[0];
-            nr[q] = nb[R];
+            nb[q] = reinterpret_cast<const unsigned *>(xr + ROWB)[(q * 2 + half) * R + wc * 32 + l32];
         }
         // tap ki reads dy row y - ki + P, or zeros beyond the image (and past
         // the slice's end)
@@ -207,9 +199,9 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
             const unsigned m0_ = __builtin_amdgcn_alignbit(v[1], v[0], 16);
             const unsigned m1_ = __builtin_amdgcn_alignbit(v[2], v[1], 16);
             const unsigned m2_ = __builtin_amdgcn_alignbit(v[3], v[2], 16);
-            b[0][q] = v4u{__builtin_amdgcn_alignbit(v[0], nl[q], 16), m0_, m1_, m2_};
+            b[0][q] = v4u{__builtin_amdgcn_alignbit(v[0], nb[q], 16), m0_, m1_, m2_};
             b[1][q] = v;
-            b[2][q] = v4u{m0_, m1_, m2_, __builtin_amdgcn_alignbit(nr[q], v[3], 16)};
+            b[2][q] = v4u{m0_, m1_, m2_, __builtin_amdgcn_alignbit(nb[q], v[3], 16)};
         }
         // the rows of step s + 1, loaded a step ago, are split and stored and
         // those of step s + 2 loaded beside the MFMAs
@@ -401,7 +393,7 @@ int wsplit_reduce(const ConvGeom &g, const WsplitPlan &pl, const float *part, fl
 
 static int wsplit_go(Wsplit &p, const WsplitPlan &pl, hipStream_t st)
 {
-    constexpr int R = 64, ROWB = 6 * R * 16, NBB = 12 * R * 4;
+    constexpr int R = 64, ROWB = 6 * R * 16, NBB = 6 * R * 4;
     p.mt = (p.F + R - 1) / R;
     p.ct = (p.C + R - 1) / R;
     p.tiles = p.mt * p.ct;

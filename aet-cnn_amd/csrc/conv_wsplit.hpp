@@ -1,4 +1,4 @@
-// Weight gradient of stride-1 "same" convolutions on the bf16 matrix cores
+// Weight gradient of 3x3 stride-1 "same" convolutions on the bf16 matrix cores
 // with every fp32 operand split exactly into three bf16 pieces
 // (conv_wsplit.hip).
 #pragma once
