@@ -32,6 +32,10 @@
 // the recomputation keeps in registers is counted beside the loop's: written
 // with indexed sums it made the kernel spill 82 registers after the loop
 // (188 us instead of 183, 62.9 MB written a launch instead of 37.7).
+// Error against 64 bits, batch 128: 128 -> 128 @ 32x32 2.5e-7 (fp32 kernel
+// 8.2e-7; 7.7e-7 with one accumulator for all products, which took 183 us),
+// 384 -> 384 @ 13x13 3.1e-7 (7.8e-7; 7.2e-7), batch 8, 64 -> 64 @ 112x112
+// 1.9e-7 (2.5e-7; 3.8e-7).
 // Partial sums laid out [tap][f][c], 32 channels a line: stored as dw is
 // ([f][c][tap], 36 bytes between lanes) the first of these took 237 us.
 #include "conv_wsplit.hpp"
@@ -170,6 +174,7 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
     // every group runs p.spw iterations, one past its last step on rows that
     // read as zero
     int y = s0 - fdiv(s0, p.dh) * p.H;
+    const v16f none = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     const unsigned frag = (half * R + l32) * 16;
     for (int s = s0; s < s0 + p.spw; ++s) {
         const char *const xr = xb + (s & 1) * (ROWB + NBB);
@@ -211,21 +216,19 @@ __global__ void __launch_bounds__(512, 2) k_conv_wsplit(Wsplit p)
         for (int i = 0; i < KS; ++i) {
             if (i + 1 < KS) load_a(i + 1);
             const v4u *ca = a[i & 1];
-            // by product over all taps: no MFMA waits for the one before it
-#define ACH_TAPS(qa, qb)                                                                  \
-    _Pragma("unroll") for (int j = 0; j < KS; ++j)                                        \
-        acc[i][j] = MFMA_BF(as_bf(ca[qa]), as_bf(b[j][qb]), acc[i][j]);
-            ACH_TAPS(2, 0) ACH_TAPS(0, 2) ACH_TAPS(1, 1) ACH_TAPS(1, 0) ACH_TAPS(0, 1)
-            ACH_TAPS(0, 0)
-#undef ACH_TAPS
-        }
+            // The matrix unit cuts off what it aligns to the largest term of a
+            // sum: with all six products added to the accumulator the sums
+            // were low by 3e-7 to 7e-7 of their size on long contractions.
+            // The five small products are summed from zero and added once.
 #pragma unroll
-        for (int i = 0; i < 6 * T; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
-            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            for (int j = 0; j < KS; ++j) {
+                v16f t = MFMA_BF(as_bf(ca[2]), as_bf(b[j][0]), none);
+                t = MFMA_BF(as_bf(ca[0]), as_bf(b[j][2]), t);
+                t = MFMA_BF(as_bf(ca[1]), as_bf(b[j][1]), t);
+                t = MFMA_BF(as_bf(ca[1]), as_bf(b[j][0]), t);
+                acc[i][j] = MFMA_BF(as_bf(ca[0]), as_bf(b[j][0]), acc[i][j]);
+                acc[i][j] += MFMA_BF(as_bf(ca[0]), as_bf(b[j][1]), t);
+            }
         }
         if (++y == p.H) y = 0;
         __syncthreads();

@@ -183,6 +183,34 @@ def test_weight_gradient(gpu, shape):
     assert np.all(abs(got - ref) <= 8 * n ** 0.5 * 2.0 ** -25 * size)
 
 
+@pytest.mark.parametrize("relu", [False, True], ids=["signed", "relu"])
+@pytest.mark.parametrize("shape,slices", [((128, 64, 32, 32, 64), 256), ((64, 250, 13, 13, 384), 10),
+                                          ((32, 512, 8, 8, 512), 4)], ids=str)
+def test_weight_gradient_error(gpu, shape, slices, relu):
+    """Relative rms error: a slice's two groups take half of its steps each,
+    and a step rounds its sums twice (leading products, small products); the
+    slices are added in four chains.  A rounding is uniform within half a
+    unit and the sums grow evenly over a chain, whose squares therefore add
+    to half the chain's length: error <=
+    2^-24 sqrt((2 steps / 2 + (slices / 4 + 4) / 2) / 3).  The mean error, to
+    which roundings in one direction would add, stays below a quarter of it."""
+    B, Cc, H, W, F = shape
+    rng = np.random.default_rng(sum(shape))
+    x = rng.standard_normal((B, Cc, H, W)).astype(np.float32)
+    if relu:
+        x = np.maximum(x, 0)
+    dy = rng.standard_normal((B, F, H, W)).astype(np.float32)
+    err = run_wgrad(gpu, x, dy, np.zeros((F, Cc, 3, 3), np.float32)).astype(np.float64)
+    ref = wgrad_ref(x.astype(np.float64), dy.astype(np.float64))
+    err -= ref
+    rms = np.sqrt((ref ** 2).mean())
+    steps = B * H * -(-W // 8) / 2 / (2 * slices)
+    limit = 2.0 ** -24 * ((steps + (slices / 4 + 4) / 2) / 3) ** 0.5
+    e = np.sqrt((err ** 2).mean()) / rms
+    print(f"{shape}: {e:.2e}, bound {limit:.2e}, mean {err.mean() / rms:.2e}")
+    assert e <= limit and abs(err.mean()) / rms <= limit / 4
+
+
 @pytest.mark.parametrize("value", [np.inf, np.nan])
 def test_weight_gradient_non_finite(gpu, value):
     """One non-finite input reaches its channel's nine taps of every filter
