@@ -50,6 +50,7 @@ constexpr int SP_CH = 16;     // input channels per chunk (one MFMA K)
 constexpr int SP_PXB = 112;   // LDS bytes per patch pixel: 3 pieces x 16 channels, padded so
                               // that eight consecutive pixels' 16-byte reads hit all banks
 constexpr int SP_BN = 128;    // output positions per workgroup
+constexpr int SP_LDS = 160 * 1024;  // LDS of a CU
 
 struct SplitFwd {
     const float *x, *wt;
@@ -478,7 +479,7 @@ SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, int fp32_splits, int 
     const int one = (pl.npx + 1) * SP_PXB;
     // two workgroups (or two K groups) share a CU's 160 KB
     pl.nbuf = 2 * one <= 80 * 1024 ? 2 : 1;
-    pl.ok = pl.kg * pl.nbuf * one <= 160 * 1024;
+    pl.ok = pl.kg * pl.nbuf * one <= SP_LDS;
     return pl;
 }
 
@@ -494,9 +495,12 @@ static int split_go(const SplitFwd &p, const SplitFwdPlan &pl, hipStream_t st)
     auto kern = epi ? &k_conv_split<WM, WN, KG, KS, TPT, true>
                     : &k_conv_split<WM, WN, KG, KS, TPT, false>;
     if (lds > 64 * 1024) {
+        // the CU's LDS, not this launch's size: the limit is the kernel's for
+        // the whole process, and another thread may launch the same kernel
+        // with a smaller patch between these two calls
         const int rc = check(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 (int)lds));
+                                                 SP_LDS));
         if (rc) return rc;
     }
     hipLaunchKernelGGL(kern, dim3(p.tiles, p.splits), dim3(64 * WM * WN * KG), lds, st, p);

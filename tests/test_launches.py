@@ -4,6 +4,28 @@ from launches import record
 WS = 1 << 40  # a workspace of any size
 
 
+def test_lds_limits_do_not_depend_on_the_layer(tmp_path):
+    """A kernel's dynamic LDS limit is process-wide: threads that run
+    different layers on the same kernel must all set the same one."""
+    shapes = [(4, 64, h, w, f, k, 1, k // 2) for f in (32, 64, 96, 128) for k, h, w in
+              ((3, 20, 78), (3, 20, 84), (3, 20, 90), (3, 20, 96), (5, 16, 44), (5, 16, 52),
+               (5, 16, 60), (5, 16, 66))]
+    calls = [[name, [{"conv": s}, "p", "p", "p", "p", WS, None]] for s in shapes
+             for name in ("ach_conv_fwd", "ach_conv_bwd_data")]
+    calls += [["ach_conv_bwd_filter", [{"conv": s}, "p", "p", "p", "p", WS, None]]
+              for s in ((128, 128, 32, 32, 128, 3, 1, 1), (64, 384, 13, 13, 384, 3, 1, 1))]
+    sizes, limits = {}, {}
+    for r in record(calls, tmp_path):
+        assert r["rc"] == 0
+        for v in r["launches"]:
+            if v["lds"] > 64 * 1024:
+                assert v["lds"] <= v["lds_limit"]
+                sizes.setdefault(v["kernel"], set()).add(v["lds"])
+                limits.setdefault(v["kernel"], set()).add(v["lds_limit"])
+    assert any(len(v) > 1 for v in sizes.values())
+    assert all(len(v) == 1 for v in limits.values())
+
+
 def test_strided_input_gradient_of_few_images(tmp_path):
     """Small grids split K: no workgroup runs a chain of more than eight
     k-tiles of 16 where the card has room for more of them."""
