@@ -276,15 +276,21 @@ __global__ void __launch_bounds__(BN_NT) k_bn_apply(
 // may be out (every thread writes only what it read, after the block's
 // barrier); xcopy / xnorm optional as in k_bn_apply.
 constexpr int BN_CH_NT = 1024;
-// Tensors of at most BN_ONE_LAUNCH values in channels of at most BN_ONE_CH take
-// one launch per direction whatever their channel count: forward 9-10 -> 5.5-7
-// us, backward 12-17 -> 7-10 us over shapes from 54 K to 1 M values (channels
-// of 441 to 16384); with 32768 values a channel's one workgroup is slower
-// (forward 10.5 against 9.6 us, backward 15.9 against 14.2).
+// Tensors of at most BN_ONE_LAUNCH values in up to BN_ONE_C channels of at most
+// BN_ONE_CH take one launch per direction: forward 9-10 -> 5.5-7 us, backward
+// 12-17 -> 7-10 us over shapes from 54 K to 1 M values (channels of 441 to
+// 16384); with 32768 values a channel's one workgroup is slower (forward 10.5
+// against 9.6 us, backward 15.9 against 14.2).  Channels run two to a CU; beyond
+// two rounds of 512 one launch is slower: 1000 channels of 784 values forward
+// 9.5 and backward 14.0 us, 10.9 and 16.1 in two launches; 1024 of 32 8.7 and
+// 11.7, 8.3 and 11.6; 4096 of 32 (a fully connected layer's) 27.0 and 37.6,
+// 14.0 and 20.2; 2048 of 200 backward 21.5, 12.8.
 constexpr long long BN_ONE_LAUNCH = 1ll << 20, BN_ONE_CH = 16384;
+constexpr int BN_ONE_C = 1000;
 static bool bn_one_launch(int batch, int c, int hw)
 {
-    return (long long)batch * hw <= BN_ONE_CH && (long long)batch * c * hw <= BN_ONE_LAUNCH;
+    return c <= BN_ONE_C && (long long)batch * hw <= BN_ONE_CH &&
+           (long long)batch * c * hw <= BN_ONE_LAUNCH;
 }
 constexpr int BN_CH_MAXV = 8;  // float4 per thread
 template <int V, bool VEC>

@@ -26,6 +26,19 @@ def test_lds_limits_do_not_depend_on_the_layer(tmp_path):
     assert all(len(v) == 1 for v in limits.values())
 
 
+def test_batchnorm_of_many_channels(tmp_path):
+    """One workgroup per channel and one launch only where they are few: a
+    fully connected layer's thousands of features of a few values take the
+    kernels that share a channel set among small workgroups."""
+    one = [(16, 72, 285), (128, 1000, 1), (4, 900, 49), (64, 1000, 16)]
+    two = [(32, 4096, 1), (128, 4096, 1), (2, 2048, 100), (32, 1001, 1)]
+    calls = [["ach_bn_bwd", ["p", *s, "p", None, *["p"] * 7, 7, "p", WS, None]] for s in one + two]
+    calls += [["ach_bn_train_fwd_from_x", ["p", "p", *s, *["p"] * 6, 7, "p", WS, None]]
+              for s in ((16, 30, 49), (32, 4096, 1), (32, 1001, 1))]
+    got = [len(r["launches"]) for r in record(calls, tmp_path)]
+    assert got == [1] * len(one) + [2] * len(two) + [1, 2, 2]
+
+
 def test_strided_input_gradient_of_few_images(tmp_path):
     """Small grids split K: no workgroup runs a chain of more than eight
     k-tiles of 16 where the card has room for more of them."""
