@@ -3563,7 +3563,7 @@ int ach_conv_bwd_data(const ach_conv_desc *d, const float *dy, const float *w, f
         const size_t fb = align256(tot * sizeof(float));
         float *part = (float *)((char *)ws + fb);
         // 1x1: the flipped k-major filter Wft[f][c] is W itself
-        if (g.KS == 1) 
+        if (g.KS == 1)
             return fwd_impl(dgrad_as_fwd(g), dy, w, dx, part, ws_bytes - fb, st, Epi(), false,
                             false);
         float *wf = (float *)ws;

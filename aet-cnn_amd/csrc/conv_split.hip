@@ -5,11 +5,10 @@
 // |a1| <= 2^-8 |a|, |a2| <= 2^-17 |a| (about).  A product a*b is taken as the
 // six piece products down to 2^-17 relative (a0b0, a0b1, a1b0, a1b1, a0b2,
 // a2b0); each is exact in the matrix unit, and what is left out (a1b2, a2b1,
-// a2b2) is below 2^-25 |ab| -- less than the rounding of one fp32 product.
-// v_mfma_f32_32x32x16_bf16 adds 16 such products and the fp32 accumulator
-// with one rounding where v_mfma_f32_32x32x2_f32 rounds after every second
-// product, and runs 16 times its rate, so the six passes cost 6/16 of the
-// fp32 instruction's matrix time.
+// a2b2) is below 2^-24 |ab|, what rounding an fp32 product can lose.  v_mfma_f32_32x32x16_bf16 adds 16 such products to the fp32
+// accumulator at once, where v_mfma_f32_32x32x2_f32 adds two, and runs 16
+// times its rate, so the six passes cost 6/16 of the fp32 instruction's matrix
+// time and the sums round an eighth as often.
 //
 // Non-finite values: an infinity (or a finite value above 2^103, which the
 // operands' scale of 2^24 takes to one) leaves non-finite residuals, so the
@@ -41,7 +40,6 @@
 // filter loads 157, without LDS reads 162 of the 178 us.
 #include "conv_split.hpp"
 #include "pieces.hpp"
-
 
 namespace ach {
 

@@ -4,9 +4,11 @@ gradient against 64-bit references where their tiles, channel chunks and K
 parts end, and infinities and NaNs.
 
 Bound, per output: the six piece products kept of a*b leave out less than
-2^-24 |ab|, and a matrix instruction adds 16 products with one rounding, so
-with K' = k*k*ceil(C/16) instructions (and a few more additions for K parts)
-|error| <= (K' + 8) 2^-24 sum |a||b|."""
+2^-24 |ab|, and a matrix instruction adds 16 products at once, so with
+K' = k*k*ceil(C/16) instructions (and a few more additions for K parts)
+|error| <= (K' + 8) 2^-24 sum |a||b|.  That bound is for indexing: over long
+sums it would hide a missing piece product, which outputs of a single product
+each (test_single_products) show at once."""
 import ctypes as C
 
 import numpy as np
@@ -62,6 +64,105 @@ def test_forward_and_input_gradient(gpu, shape):
     ref = refs64.dgrad_ref(dy, w, x.shape, 1, p)
     mag = refs64.dgrad_ref(abs(dy), abs(w), x.shape, 1, p)
     assert np.all(abs(dx.numpy() - ref) <= bound(mag, k, F))
+
+
+# the piece products left out (below 2^-24 of a product, and 2^-10 of that),
+# the rounding of the sum of the small ones and that of the result
+ONE_PRODUCT = 2.1 * 2.0 ** -24
+
+
+def one_each(rng, groups, members):
+    """A member for each group, every member in turn in a random order."""
+    return np.resize(rng.permutation(members), groups)
+
+
+@pytest.mark.parametrize("shape", [SHAPES[1], SHAPES[3], SHAPES[4], SHAPES[5], SHAPES[12],
+                                   SHAPES[14], SHAPES[15], (128, 64, 13, 13, 320, 3, 1)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_single_products(gpu, shape):
+    """Filters with one nonzero weight for each output (and, for the input
+    gradient, for each input channel): every sum is one product, which all
+    six piece products make exact to ONE_PRODUCT and any five do not."""
+    B, Cc, H, W, F, k, p = shape
+    rng = np.random.default_rng(sum(shape))
+    x = rng.standard_normal((B, Cc, H, W)).astype(np.float32)
+    oh, ow = H + 2 * p - k + 1, W + 2 * p - k + 1
+    dy = rng.standard_normal((B, F, oh, ow)).astype(np.float32)
+    d = aetcnn.ConvDesc(B, Cc, H, W, F, k, 1, p)
+    nb = max(gpu.ach_conv_fwd_workspace(C.byref(d)), gpu.ach_conv_bwd_data_workspace(C.byref(d)))
+    ws, dx_, ddy, y, dx = D(nb // 4 + 64), D.from_numpy(x), D.from_numpy(dy), D(dy.shape), D(x.shape)
+    for fwd in (True, False):
+        w = np.zeros((F, Cc, k, k), np.float32)
+        n, m = (F, Cc) if fwd else (Cc, F)
+        at = one_each(rng, n, m * k * k)
+        a, i, j = at // (k * k), at // k % k, at % k
+        v = rng.standard_normal(n).astype(np.float32)
+        if fwd:
+            w[np.arange(F), a, i, j] = v
+        else:
+            w[a, np.arange(Cc), i, j] = v
+        dw = D.from_numpy(w)
+        if fwd:
+            check(gpu.ach_conv_fwd(C.byref(d), dx_.ptr, dw.ptr, y.ptr, ws.ptr, nb, None))
+            got, ref = y.numpy(), refs64.conv_ref(x, w, 1, p)
+        else:
+            check(gpu.ach_conv_bwd_data(C.byref(d), ddy.ptr, dw.ptr, dx.ptr, ws.ptr, nb, None))
+            got, ref = dx.numpy(), refs64.dgrad_ref(dy, w, x.shape, 1, p)
+        assert np.all(abs(got - ref) <= ONE_PRODUCT * abs(ref)), fwd
+
+
+def test_single_products_of_weight_gradients(gpu):
+    """One nonzero delta for each filter."""
+    for shape in WGRAD:
+        B, Cc, H, W, F = shape
+        rng = np.random.default_rng(sum(shape))
+        x = rng.standard_normal((B, Cc, H, W)).astype(np.float32)
+        dy = np.zeros((B, F, H, W), np.float32)
+        at = one_each(rng, F, B * H * W)
+        b, i, j = at // (H * W), at // W % H, at % W
+        v = rng.standard_normal(F).astype(np.float32)
+        dy[b, np.arange(F), i, j] = v
+        got = run_wgrad(gpu, x, dy, np.zeros((F, Cc, 3, 3), np.float32))
+        xp = np.pad(x, ((0, 0), (0, 0), (1, 1), (1, 1))).astype(np.float64)
+        ref = np.stack([np.stack([xp[b, :, i + ki, j + kj] for kj in range(3)], -1)
+                        for ki in range(3)], -2) * v.astype(np.float64)[:, None, None, None]
+        assert np.all(abs(got - ref) <= ONE_PRODUCT * abs(ref)), shape
+
+
+@pytest.mark.parametrize("B,K,F", [(33, 128, 128), (64, 300, 130), (130, 520, 256),
+                                   (70, 2900, 2890)], ids=str)
+def test_single_products_fully_connected(gpu, B, K, F):
+    rng = np.random.default_rng(B + K + F)
+    x = rng.standard_normal((B, K)).astype(np.float32)
+    dy = rng.standard_normal((B, F)).astype(np.float32)
+    d = aetcnn.ConvDesc(B, K, 1, 1, F, 1, 1, 0)
+    r = C.byref(d)
+    nb = max(gpu.ach_conv_fwd_workspace(r), gpu.ach_conv_bwd_data_workspace(r),
+             gpu.ach_conv_bwd_filter_workspace(r))
+    ws, dx_, ddy = D(nb // 4 + 64), D.from_numpy(x), D.from_numpy(dy)
+    y, dx, g = D((B, F)), D((B, K)), D((F, K))
+    w = np.zeros((F, K), np.float32)
+    at = one_each(rng, F, K)
+    w[np.arange(F), at] = rng.standard_normal(F)
+    dw = D.from_numpy(w)
+    check(gpu.ach_conv_fwd(r, dx_.ptr, dw.ptr, y.ptr, ws.ptr, nb, None))
+    ref = x[:, at].astype(np.float64) * w[np.arange(F), at]
+    assert np.all(abs(y.numpy() - ref) <= ONE_PRODUCT * abs(ref))
+    w = np.zeros((F, K), np.float32)
+    at = one_each(rng, K, F)
+    w[at, np.arange(K)] = rng.standard_normal(K)
+    dw = D.from_numpy(w)
+    check(gpu.ach_conv_bwd_data(r, ddy.ptr, dw.ptr, dx.ptr, ws.ptr, nb, None))
+    ref = dy[:, at].astype(np.float64) * w[at, np.arange(K)]
+    assert np.all(abs(dx.numpy() - ref) <= ONE_PRODUCT * abs(ref))
+    one = np.zeros((B, F), np.float32)
+    at = one_each(rng, F, B)
+    one[at, np.arange(F)] = dy[at, np.arange(F)]
+    g.zero()
+    done = D.from_numpy(one)
+    check(gpu.ach_conv_bwd_filter(r, dx_.ptr, done.ptr, g.ptr, ws.ptr, nb, None))
+    ref = dy[at, np.arange(F)].astype(np.float64)[:, None] * x[at]
+    assert np.all(abs(g.numpy() - ref) <= ONE_PRODUCT * abs(ref))
 
 
 @pytest.mark.parametrize("shape", [(2, 32, 9, 9, 48, 3, 1), (64, 128, 8, 8, 128, 3, 1)],
