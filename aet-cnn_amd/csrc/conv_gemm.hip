@@ -2889,7 +2889,7 @@ static size_t fp32_part_bytes(const ConvGeom &g, bool kg_ok = true)
 static size_t fwd_part_bytes(const ConvGeom &g, bool kg_ok = true)
 {
     const FwdPlan pl = fwd_plan(g, kg_ok);
-    const SplitFwdPlan sp = split_fwd_plan(g, kg_ok, pl.pslices(), 1 << 30);
+    const SplitFwdPlan sp = split_fwd_plan(g, kg_ok, pl.splits, pl.pslices(), 1 << 30);
     const size_t need = fp32_part_bytes(g, kg_ok);
     const int slices = fc_geom(g) ? fc_split_slices(g.B, g.F, g.C, 1 << 30) : sp.ok ? sp.splits : 0;
     if (slices <= 1) return need;
@@ -3025,7 +3025,8 @@ static int fwd_impl(const ConvGeom &g, const float *x, const float *w, float *y,
                           : fwd_small_k_launch<false>(g, x, w, y, e, w_nat, st);
     const FwdPlan pl = fwd_plan(g, kg_ok);
     const size_t room = part ? part_bytes / ((size_t)g.F * g.B * g.OH * g.OW * sizeof(float)) : 0;
-    SplitFwdPlan sp = split_fwd_plan(g, kg_ok, pl.pslices(), room > 1024 ? 1024 : (int)room);
+    SplitFwdPlan sp = split_fwd_plan(g, kg_ok, pl.splits, pl.pslices(),
+                                     room > 1024 ? 1024 : (int)room);
     sp.ok = sp.ok && pieces;
     const int fc = pieces && fc_geom(g)
                        ? fc_split_slices(g.B, g.F, g.C, room > 1024 ? 1024 : (int)room) : 0;

@@ -15,10 +15,11 @@ struct SplitFwdPlan {
     int splits;     // grid slices of K (each kg groups wide); partials if > 1
 };
 
-// kg_ok: the call may run two K groups per workgroup; fp32_splits: the slices
-// of partial sums the fp32 plan takes; room: those that the caller's workspace
-// holds
-SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, int fp32_splits, int room);
+// kg_ok: the call may run two K groups per workgroup; fp32_parts: the parts
+// that the fp32 plan adds up; fp32_splits: the slices of partial sums it
+// writes; room: those that the caller's workspace holds
+SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, int fp32_parts, int fp32_splits,
+                            int room);
 
 // y (or part[z][m][n] when pl.splits > 1) = conv(x, wt); wt k-major Wt[K][M].
 // The epilogue e is applied when K is not split over the grid.

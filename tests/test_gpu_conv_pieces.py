@@ -165,6 +165,35 @@ def test_single_products_fully_connected(gpu, B, K, F):
     assert np.all(abs(g.numpy() - ref) <= ONE_PRODUCT * abs(ref))
 
 
+@pytest.mark.parametrize("shape", [
+    (8, 128, 20, 56, 96, 5, 2),    # fp32: 13 parts of K
+    (8, 128, 20, 66, 96, 5, 2),
+    (2, 512, 10, 10, 64, 5, 2),    # few tiles, long sums
+    (4, 500, 12, 12, 30, 3, 1),
+    (8, 512, 8, 8, 512, 3, 1),
+], ids=lambda s: "x".join(map(str, s)))
+def test_error_against_fp32_form(gpu, shape):
+    """No further from 64 bits than the fp32 form of the same call, which adds
+    up K in many parts on small grids."""
+    B, Cc, H, W, F, k, p = shape
+    rng = np.random.default_rng(sum(shape))
+    x = rng.standard_normal((B, Cc, H, W)).astype(np.float32)
+    w = rng.standard_normal((F, Cc, k, k)).astype(np.float32)
+    d = aetcnn.ConvDesc(B, Cc, H, W, F, k, 1, p)
+    nb = gpu.ach_conv_fwd_workspace(C.byref(d))
+    ws, dx, dw, wt = D(nb // 4 + 64), D.from_numpy(x), D.from_numpy(w), D(w.size)
+    job = aetcnn.FilterJob(d, dw.ptr, wt.ptr, None)
+    check(gpu.ach_conv_prepare_filters(1, C.byref(job), None))
+    a, b = D((B, F, H, W)), D((B, F, H, W))
+    check(gpu.ach_conv_fwd_prepared(C.byref(d), dx.ptr, wt.ptr, a.ptr, ws.ptr, nb, None))
+    check(gpu.ach_conv_fwd_train_prepared(C.byref(d), dx.ptr, wt.ptr, None, aetcnn.LINEAR, b.ptr,
+                                          ws.ptr, nb, None))
+    ref = refs64.conv_ref(x, w, 1, p)
+    e = [rel_rms(t.numpy(), ref) for t in (a, b)]
+    print(f"{shape}: {e[0]:.2e}, fp32 {e[1]:.2e}")
+    assert e[0] <= e[1]
+
+
 @pytest.mark.parametrize("shape", [(2, 32, 9, 9, 48, 3, 1), (64, 128, 8, 8, 128, 3, 1)],
                          ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, np.float32(3.4e38)])
