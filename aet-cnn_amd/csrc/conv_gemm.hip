@@ -31,6 +31,7 @@
 #include "conv_wsplit.hpp"
 #include "fc_split.hpp"
 
+#include <math.h>
 #include <type_traits>
 
 namespace ach {
@@ -3710,6 +3711,25 @@ int ach_conv_bwd_data_prepared(const ach_conv_desc *d, const float *dy, const fl
                     Epi(), false, false);
 }
 
+// the three-piece weight gradient's plan beside an fp32 plan of that many
+// parts, whose reduction adds them up in groups from two groups on.  The fp32
+// kernel's time, fitted to 900 layers (within a tenth on eight of ten): whole
+// tiles and k-tiles at 138 TFLOP/s, the partial sums at 7 TB/s and 13 us.
+// (349 -> 463 @ 43x43, batch 10: 679 us, 692 measured; 505 -> 139 @ 27x15,
+// batch 88: 649, 640; 368 -> 464 @ 42x42, batch 3: 368, 423.)
+static WsplitPlan wgrad_pieces_plan(const ConvGeom &g, int bm, int bn, int splits, int room)
+{
+    Fp32Wgrad f;
+    f.parts = splits;
+    f.adds = splits > 2 * SPLIT_GROUP
+                 ? SPLIT_GROUP + (splits + SPLIT_GROUP - 1) / SPLIT_GROUP : splits;
+    const double n = (double)g.C * g.KS * g.KS, k = ((double)g.B * g.OH * g.OW + 15) / 16;
+    const double rows = (double)((g.F + bm - 1) / bm) * bm, cols = ceil(n / bn) * bn;
+    f.us = 13.0 + 2.0 * 16 * floor(k) * rows * cols / 138e6 +
+           (splits > 1 ? splits * n * g.F * 4 * 2 / 7e6 : 0.0);
+    return wsplit_plan(g, f, room);
+}
+
 // bytes that the fp32 weight gradient needs
 static size_t fp32_wgrad_bytes(const ConvGeom &g)
 {
@@ -3728,7 +3748,10 @@ size_t ach_conv_bwd_filter_workspace(const ach_conv_desc *d)
     const ConvGeom g = geom(d);
     if (conv_xy(d)) return xy_col_bytes(g);
     const size_t need = fp32_wgrad_bytes(g);
-    const WsplitPlan wp = wsplit_plan(g, 1 << 30);
+    const int bm = wgrad_bm(g), bn = wgrad_bn(g);
+    int splits, kchunk;
+    wgrad_split(g, bm, bn, splits, kchunk);
+    const WsplitPlan wp = wgrad_pieces_plan(g, bm, bn, splits, 1 << 30);
     if (!wp.ok) return need;
     const size_t n = (size_t)wp.splits * g.F * g.C * g.KS * g.KS * sizeof(float);
     return n > need ? n : need;
@@ -3766,7 +3789,7 @@ static int bwd_filter(const ach_conv_desc *d, const float *x, const float *dy, f
     bool done = false;  // the update was applied in the GEMM's epilogue
     // the three-piece kernel, with the slices that the workspace holds
     const size_t held = ws ? ws_bytes / ((size_t)g.F * g.C * g.KS * g.KS * sizeof(float)) : 0;
-    const WsplitPlan wp = wsplit_plan(g, held > 1 << 20 ? 1 << 20 : (int)held);
+    const WsplitPlan wp = wgrad_pieces_plan(g, bm, bn, splits, held > 1 << 20 ? 1 << 20 : (int)held);
     if (wp.ok) {
         rc = wsplit_launch(g, wp, x, dy, part, st);
         return rc ? rc : wsplit_reduce(g, wp, part, dw, sgd, st);

@@ -417,7 +417,13 @@ static void split_patch(const ConvGeom &g, long long &npx, long long &nreal)
     nreal = real * g.W;
 }
 
-SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, int fp32_parts, int fp32_splits, int room)
+// 72 steps, 128 -> 128 @ 32x32: 2.0e-7, after a relu 1.5e-7.  (128 -> 96 5x5 at
+// 20x56, batch 8, in one chain of 200 steps was at 3.4e-7, the fp32 kernel with
+// 13 parts at 2.7e-7.)
+constexpr StepError kStepError = {1.8, 1.25};
+
+SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, int fp32_parts, int fp32_splits,
+                            int room)
 {
     SplitFwdPlan pl{};
     pl.ok = false;
@@ -457,13 +463,9 @@ SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, int fp32_parts, int f
                 if (s * kg > nchunk || (s > 1 && tiles * s > 2048)) break;
                 const int cps = (nchunk + s * kg - 1) / (s * kg);
                 const int splits = (nchunk + cps * kg - 1) / (cps * kg);
-                // The error of a chain goes with the root of its length: 2.0e-7
-                // for 72 steps of 16 products here, 6.0e-7 for 1152 products
-                // on the fp32 instructions.  Nine times the fp32 plan's parts
-                // is what one here may hold to be no further from 64 bits:
-                // 128 -> 96 5x5 at 20x56, batch 8, in one chain of 200 steps
-                // was (3.4e-7, 2.7e-7 in 13 fp32 parts).
-                if (9 * splits * kg < fp32_parts) continue;
+                if (!no_more_error(kStepError, cps * g.KS * g.KS, splits * kg,
+                                   (double)g.C * g.KS * g.KS / fp32_parts, fp32_parts))
+                    continue;
                 if (splits > 1 && (splits > room || (splits > fp32_splits && big < 128))) continue;
                 const long long wgs = tiles * splits;
                 const long long full = wgs >> (kg == 2 ? 8 : 9), rest = wgs & (kg == 2 ? 255 : 511);

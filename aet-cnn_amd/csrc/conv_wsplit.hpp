@@ -13,8 +13,15 @@ struct WsplitPlan {
     int spw;     // K steps per (slice, group)
 };
 
+// what the fp32 kernel would do: parts of K, the additions that one of them
+// goes through when they are added up (in groups), and its modelled time
+struct Fp32Wgrad {
+    int parts, adds;
+    double us;
+};
+
 // room: slices of partial sums that the caller's workspace holds
-WsplitPlan wsplit_plan(const ConvGeom &g, int room);
+WsplitPlan wsplit_plan(const ConvGeom &g, const Fp32Wgrad &fp32, int room);
 
 // part[z][ki*k + kj][f][c] = the slice's sums of dy * shifted x
 int wsplit_launch(const ConvGeom &g, const WsplitPlan &pl, const float *x, const float *dy,
