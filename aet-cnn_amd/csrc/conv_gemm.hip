@@ -3714,9 +3714,10 @@ int ach_conv_bwd_data_prepared(const ach_conv_desc *d, const float *dy, const fl
 // the three-piece weight gradient's plan beside an fp32 plan of that many
 // parts, whose reduction adds them up in groups from two groups on.  The fp32
 // kernel's time, fitted to 900 layers (within a tenth on eight of ten): whole
-// tiles and k-tiles at 138 TFLOP/s, the partial sums at 7 TB/s and 13 us.
-// (349 -> 463 @ 43x43, batch 10: 679 us, 692 measured; 505 -> 139 @ 27x15,
-// batch 88: 649, 640; 368 -> 464 @ 42x42, batch 3: 368, 423.)
+// tiles and k-tiles at 139 TFLOP/s (134 in the position order), the partial
+// sums at 7 TB/s and 13 us.  (349 -> 463 @ 43x43, batch 10: 692 us, 692
+// measured; 505 -> 139 @ 27x15, batch 88: 667, 640; 368 -> 464 @ 42x42, batch 3:
+// 374, 423.)
 static WsplitPlan wgrad_pieces_plan(const ConvGeom &g, int bm, int bn, int splits, int room)
 {
     Fp32Wgrad f;
@@ -3725,7 +3726,7 @@ static WsplitPlan wgrad_pieces_plan(const ConvGeom &g, int bm, int bn, int split
                  ? SPLIT_GROUP + (splits + SPLIT_GROUP - 1) / SPLIT_GROUP : splits;
     const double n = (double)g.C * g.KS * g.KS, k = ((double)g.B * g.OH * g.OW + 15) / 16;
     const double rows = (double)((g.F + bm - 1) / bm) * bm, cols = ceil(n / bn) * bn;
-    f.us = 13.0 + 2.0 * 16 * floor(k) * rows * cols / 138e6 +
+    f.us = 13.0 + 2.0 * 16 * floor(k) * rows * cols / (wgrad_chunked(g) ? 139e6 : 134e6) +
            (splits > 1 ? splits * n * g.F * 4 * 2 / 7e6 : 0.0);
     return wsplit_plan(g, f, room);
 }

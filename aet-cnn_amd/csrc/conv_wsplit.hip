@@ -434,16 +434,15 @@ WsplitPlan wsplit_plan(const ConvGeom &g, const Fp32Wgrad &fp32, int room)
     const long long S = units * g.H;
     if (S >= (1ll << 26)) return pl;
     const long long tiles = (long long)((g.F + 63) / 64) * ((g.C + 63) / 64);
-    // Time model (us), fitted to a sweep of layer shapes: a step of the two
-    // groups' eight waves; more where the rows are not whole segments, and
-    // where a line of memory holds several units' segments of an image pair,
-    // which are read far apart (the line comes from HBM for each); the
-    // partial sums written and read; and prologue, exchange and reduction.
-    const double step = pair && nu >= 3 ? (nu >= 5 ? 4.4 : 3.5) : (g.W % 8 ? 2.7 : 2.4);
+    // Time model (us), fitted to 185 of 900 layer shapes that run here: a step
+    // of the two groups' eight waves, 2.1-2.4 where rows are whole segments,
+    // 2.5-2.9 where they are not, 3.3-4.5 and 4.0-5.4 where, besides, a line of
+    // memory holds three or five segments of an image pair, which are read far
+    // apart (the line comes from HBM for each); the partial sums written and
+    // read; and prologue, exchange and reduction.
+    const double step = g.W % 8 == 0 ? 2.4 : !pair || nu < 3 ? 2.8 : nu < 5 ? 4.2 : 4.8;
     const double mn4 = (double)g.F * g.C * g.KS * g.KS * 4;
-    // (both models are within a tenth on nine layers of ten: the plan has to
-    // promise a tenth for the fp32 kernel to give way)
-    const double limit = 0.9 * fp32.us;
+    const double limit = 0.95 * fp32.us;
     if (limit < 12.0 + 4 * step + 4.0) return pl;  // the shortest plan is no faster
     auto precise = [&](int s, long long spw) {
         return no_more_error(kStepError, (double)spw, s / 4.0 + 4,
