@@ -2663,6 +2663,11 @@ struct FwdPlan {
     int kg;  // K slices per workgroup (kg == splits: no partial sums)
     // partial-sum slices written (each workgroup adds its kg slices first)
     int pslices() const { return splits / kg; }
+    Fp32Fwd as_fp32(const ConvGeom &g) const
+    {
+        const long long n = (long long)g.B * g.OH * g.OW;
+        return {splits, pslices(), (int)((g.F + bm - 1) / bm * ((n + 127) / 128)), kchunk / bk};
+    }
 };
 
 // a 1x1 convolution of a 1x1 input (the fully connected layers once geom()
@@ -2890,7 +2895,7 @@ static size_t fp32_part_bytes(const ConvGeom &g, bool kg_ok = true)
 static size_t fwd_part_bytes(const ConvGeom &g, bool kg_ok = true)
 {
     const FwdPlan pl = fwd_plan(g, kg_ok);
-    const SplitFwdPlan sp = split_fwd_plan(g, kg_ok, pl.splits, pl.pslices(), 1 << 30);
+    const SplitFwdPlan sp = split_fwd_plan(g, kg_ok, pl.as_fp32(g), 1 << 30);
     const size_t need = fp32_part_bytes(g, kg_ok);
     const int slices = fc_geom(g) ? fc_split_slices(g.B, g.F, g.C, 1 << 30) : sp.ok ? sp.splits : 0;
     if (slices <= 1) return need;
@@ -3026,8 +3031,7 @@ static int fwd_impl(const ConvGeom &g, const float *x, const float *w, float *y,
                           : fwd_small_k_launch<false>(g, x, w, y, e, w_nat, st);
     const FwdPlan pl = fwd_plan(g, kg_ok);
     const size_t room = part ? part_bytes / ((size_t)g.F * g.B * g.OH * g.OW * sizeof(float)) : 0;
-    SplitFwdPlan sp = split_fwd_plan(g, kg_ok, pl.splits, pl.pslices(),
-                                     room > 1024 ? 1024 : (int)room);
+    SplitFwdPlan sp = split_fwd_plan(g, kg_ok, pl.as_fp32(g), room > 1024 ? 1024 : (int)room);
     sp.ok = sp.ok && pieces;
     const int fc = pieces && fc_geom(g)
                        ? fc_split_slices(g.B, g.F, g.C, room > 1024 ? 1024 : (int)room) : 0;

@@ -422,8 +422,36 @@ static void split_patch(const ConvGeom &g, long long &npx, long long &nreal)
 // 13 parts at 2.7e-7.)
 constexpr StepError kStepError = {1.8, 1.25};
 
-SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, int fp32_parts, int fp32_splits,
-                            int room)
+// Up to 32 filters a workgroup has little work for its loads, and small grids
+// of them can be slower than the fp32 kernel's: 144 -> 16 5x5 at 45x32, one
+// image, 21.6 us, 14.4 on fp32.  Both times (us) by models fitted to 4700 such
+// layers, within 6% on eight of ten (one set of constants for 3x3, one for
+// 5x5): a step of a chunk (or k-tile) with one workgroup on every CU and with
+// more, the partial sums in MB, workgroups in thousands.
+struct NarrowTime {
+    double fix, one, more, split, mb, wgs;
+};
+constexpr NarrowTime kNarrowPieces[2] = {{6.1, 2.4, 3.9, 2.9, 0.19, 3.2}, {5.9, 2.1, 3.3, 2.5, 0.25, 3.1}};
+constexpr NarrowTime kNarrowFp32[2] = {{4.9, 0.59, 0.28, 2.9, 0.20, 2.3}, {4.7, 0.96, 0.34, 1.4, 0.29, 3.9}};
+
+static bool narrow_pays(const ConvGeom &g, const SplitFwdPlan &pl, const Fp32Fwd &fp32)
+{
+    const double mn = (double)g.F * g.B * g.OH * g.OW * 4e-6, taps = g.KS * g.KS / 9.0;
+    const int nchunk = (g.C + SP_CH - 1) / SP_CH, cps = (nchunk + pl.splits - 1) / pl.splits;
+    const long long wgs = ((long long)g.B * g.OH * g.OW + SP_BN - 1) / SP_BN * pl.splits;
+    const NarrowTime &p = kNarrowPieces[g.KS == 5], &f = kNarrowFp32[g.KS == 5];
+    const long long full = wgs / 512, rest = wgs % 512;
+    double tp = p.fix + cps * taps * (full * p.more + (rest > 256 ? p.more : rest ? p.one : 0.0)) +
+                p.wgs * wgs / 1000;
+    if (pl.splits > 1) tp += p.split + p.mb * (2 * pl.splits + 1) * mn;
+    const double wf = (double)fp32.tiles * fp32.parts;
+    double tf = f.fix + fp32.ktiles * (f.one + f.more * (wf > 256 ? wf / 256 - 1 : 0.0)) +
+                f.wgs * wf / 1000;
+    if (fp32.slices > 1) tf += f.split + f.mb * (2 * fp32.slices + 1) * mn;
+    return tp < tf;
+}
+
+SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, const Fp32Fwd &fp32, int room)
 {
     SplitFwdPlan pl{};
     pl.ok = false;
@@ -464,9 +492,9 @@ SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, int fp32_parts, int f
                 const int cps = (nchunk + s * kg - 1) / (s * kg);
                 const int splits = (nchunk + cps * kg - 1) / (cps * kg);
                 if (!no_more_error(kStepError, cps * g.KS * g.KS, splits * kg,
-                                   (double)g.C * g.KS * g.KS / fp32_parts, fp32_parts))
+                                   (double)g.C * g.KS * g.KS / fp32.parts, fp32.parts))
                     continue;
-                if (splits > 1 && (splits > room || (splits > fp32_splits && big < 128))) continue;
+                if (splits > 1 && (splits > room || (splits > fp32.slices && big < 128))) continue;
                 const long long wgs = tiles * splits;
                 const long long full = wgs >> (kg == 2 ? 8 : 9), rest = wgs & (kg == 2 ? 255 : 511);
                 double t = full * cps * paired;
@@ -486,7 +514,7 @@ SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, int fp32_parts, int f
     const int one = (pl.npx + 1) * SP_PXB;
     // two workgroups (or two K groups) share a CU's 160 KB
     pl.nbuf = 2 * one <= 80 * 1024 ? 2 : 1;
-    pl.ok = pl.kg * pl.nbuf * one <= SP_LDS;
+    pl.ok = pl.kg * pl.nbuf * one <= SP_LDS && (M > 32 || narrow_pays(g, pl, fp32));
     return pl;
 }
 

@@ -15,11 +15,15 @@ struct SplitFwdPlan {
     int splits;     // grid slices of K (each kg groups wide); partials if > 1
 };
 
-// kg_ok: the call may run two K groups per workgroup; fp32_parts: the parts
-// that the fp32 plan adds up; fp32_splits: the slices of partial sums it
-// writes; room: those that the caller's workspace holds
-SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, int fp32_parts, int fp32_splits,
-                            int room);
+// what the fp32 kernel would do: parts of K that it adds up, slices of partial
+// sums that it writes, tiles of its grid and k-tiles of a part
+struct Fp32Fwd {
+    int parts, slices, tiles, ktiles;
+};
+
+// kg_ok: the call may run two K groups per workgroup; room: the slices of
+// partial sums that the caller's workspace holds
+SplitFwdPlan split_fwd_plan(const ConvGeom &g, bool kg_ok, const Fp32Fwd &fp32, int room);
 
 // y (or part[z][m][n] when pl.splits > 1) = conv(x, wt); wt k-major Wt[K][M].
 // The epilogue e is applied when K is not split over the grid.
