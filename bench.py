@@ -40,16 +40,21 @@ SWEEP = [  # config 1: (C_in, C_out, H, k, pad)
     (256, 512, 8, 3, 1), (512, 512, 8, 3, 1), (512, 10, 8, 1, 0),
 ]
 # Kernel probes, each one config-1 / config-3 layer pass launched back to
-# back on its own stream: the three-piece convolution (input gradients and
-# operation-level forwards run it) and the three-piece weight gradient.
+# back on its own stream: the training forward (fp32 instructions), the input
+# gradient and the weight gradient (three bf16 pieces), as a training step runs
+# them.
 PROBES = {
-    "fwd": dict(shape=(256, 256, 16, 3, 1), op="fwd",
-                kernel="k_conv_split<4, 1, 1, 3, 2, false> (three-piece bf16 convolution; the "
-                       "stride-1 input gradient runs the same kernel)"),
-    "wgrad": dict(shape=(128, 128, 32, 3, 1), op="wgrad",
+    "fwd": dict(shape=(256, 256, 16, 3, 1), op="fwd", match="k_mfma_gemm",
+                peak=MFMA_FP32_PEAK_TFLOPS,
+                kernel="k_mfma_gemm<FwdProblem<128, BIm2col3F, true, false>, 2> (training "
+                       "forward implicit GEMM, two K groups per workgroup)"),
+    "dgrad": dict(shape=(256, 256, 16, 3, 1), op="dgrad", match="k_conv_split",
+                  peak=MFMA_PIECES_PEAK_TFLOPS,
+                  kernel="k_conv_split<4, 1, 1, 3, 2, false> (three-piece bf16 convolution)"),
+    "wgrad": dict(shape=(128, 128, 32, 3, 1), op="wgrad", match="k_conv_wsplit",
+                  peak=MFMA_PIECES_PEAK_TFLOPS,
                   kernel="k_conv_wsplit<true> (three-piece bf16 weight gradient)"),
 }
-PROBE_KERNELS = ("k_conv_split", "k_conv_wsplit")
 CALIB_FLOATS = 1 << 26  # the 256 MiB copy-calibration dispatch
 
 
@@ -271,27 +276,31 @@ def probe_setup(aetcnn, which, batch):
     rng = np.random.default_rng(1)
     xh, wh, dyh = config1_inputs(rng, batch, ci, co, hw, k, p)
     x, w, dy = D.from_numpy(xh), D.from_numpy(wh), D.from_numpy(dyh)
-    y, dw = D(dyh.shape), D(wh.shape)
-    wt = D(wh.shape)
-    wsz = max(ops.ach_conv_fwd_workspace(C.byref(d)),
+    y, dx, dw = D(dyh.shape), D(xh.shape), D(wh.shape)
+    wt, wft = D(wh.shape), D(wh.shape)
+    wsz = max(ops.ach_conv_fwd_workspace(C.byref(d)), ops.ach_conv_bwd_data_workspace(C.byref(d)),
               ops.ach_conv_bwd_filter_workspace(C.byref(d)), 256)
     ws = D(wsz // 4 + 64)
+    # the k-major filters made once, as the network does once per step for all
+    # its layers: each call of the first two is then the GEMM launch alone
+    job = aetcnn.FilterJob(d, w.ptr, wt.ptr, wft.ptr)
+    aetcnn.check(ops.ach_conv_prepare_filters(1, C.byref(job), stream), "prepare")
     if PROBES[which]["op"] == "fwd":
-        # the k-major filter made once, as the network does once per step
-        # for all its layers: each call is then the GEMM launch alone
-        job = aetcnn.FilterJob(d, w.ptr, wt.ptr, None)
-        aetcnn.check(ops.ach_conv_prepare_filters(1, C.byref(job), stream), "prepare")
-
         def call():
-            aetcnn.check(ops.ach_conv_fwd_prepared(C.byref(d), x.ptr, wt.ptr, y.ptr, ws.ptr, wsz,
-                                                   stream))
+            aetcnn.check(ops.ach_conv_fwd_train_prepared(C.byref(d), x.ptr, wt.ptr, None,
+                                                         aetcnn.LINEAR, y.ptr, ws.ptr, wsz,
+                                                         stream))
+    elif PROBES[which]["op"] == "dgrad":
+        def call():
+            aetcnn.check(ops.ach_conv_bwd_data_prepared(C.byref(d), dy.ptr, w.ptr, wft.ptr, dx.ptr,
+                                                        ws.ptr, wsz, stream))
     else:
         def call():
             aetcnn.check(ops.ach_conv_bwd_filter(C.byref(d), x.ptr, dy.ptr, dw.ptr, ws.ptr, wsz,
                                                  stream))
 
     def free():
-        for a in (x, w, dy, y, dw, ws, wt):
+        for a in (x, w, dy, y, dx, dw, ws, wt, wft):
             a.free()
         ops.ach_stream_destroy(stream)
     oh = hw + 2 * p - k + 1
@@ -301,11 +310,10 @@ def probe_setup(aetcnn, which, batch):
 
 def roofline_phase(aetcnn, which, batch, reps):
     """A probe launched `reps` times back to back with HIP events around the
-    run on the probe's stream.  The forward call is the GEMM launch alone
-    (ach_conv_fwd_prepared on a k-major filter made once: 512 workgroups of
-    128 x 128 tiles), so the average is that kernel's; the weight-gradient
-    call is the GEMM and its fixed-order reduction, whose average is the
-    whole call."""
+    run on the probe's stream.  The forward and input-gradient calls are the
+    GEMM launch alone (k-major filters made once: 512 workgroups over 128 x
+    128 tiles), so the average is that kernel's; the weight-gradient call is
+    the GEMM and its fixed-order reduction, whose average is the whole call."""
     ops = aetcnn.ops()
     call, stream, free, flop, shape = probe_setup(aetcnn, which, batch)
     ms = time_launch(ops, stream, call, reps)
@@ -379,7 +387,7 @@ def traffic_phase(which, calls=3, timeout=120):
             expect_kib = CALIB_FLOATS * 4 / 1024.0
             scale[ctr] = expect_kib / disp[cal[0]][1]
             after = [i for i in ids if i > cal[0]]
-            ngemm = sum(1 for i in after if any(k in disp[i][0] for k in PROBE_KERNELS))
+            ngemm = sum(1 for i in after if PROBES[which]["match"] in disp[i][0])
             if ngemm != calls:
                 return None, f"{ctr}: expected {calls} GEMM dispatches, found {ngemm}"
             tot = 0.0
@@ -401,8 +409,9 @@ def traffic_phase(which, calls=3, timeout=120):
 
 
 def algorithmic_bytes(which, batch=128):
-    """Operands each probe call must move at least once: conv forward reads
-    x and W and writes y; the weight gradient reads x and dy and writes dW."""
+    """Operands each probe call must move at least once: the forward reads x
+    and W and writes y, the input gradient reads dy and W and writes dx, the
+    weight gradient reads x and dy and writes dW."""
     ci, co, hw, k, p = PROBES[which]["shape"]
     oh = hw + 2 * p - k + 1
     x, w, y = batch * ci * hw * hw, co * ci * k * k, batch * co * oh * oh
@@ -706,7 +715,7 @@ def main():
                 ms_per_step=round(oms, 4), images_per_s=round(o["batch"] * args.steps / o["wall_s"], 1),
                 gpu_ms_per_step=round(o["gpu_ms"] / args.steps, 4), batch=o["batch"],
                 steps=args.steps, warmup=args.warmup, conv_gflop_per_step=round(o["gflop_step"], 2),
-                conv_tflops=round(otf, 3), frac_of_fp32_mfma_peak=round(otf / MFMA_FP32_PEAK_TFLOPS, 4),
+                conv_tflops=round(otf, 3),
                 loss_first_last=[round(o["first_loss"], 5), round(o["loss"], 5)])
             log(f"{name} b{o['batch']}: {oms:.3f} ms/step, "
                 f"{other_steps[name + '_step']['images_per_s']} img/s, conv {otf:.2f} TFLOP/s")
@@ -737,8 +746,8 @@ def main():
         else:
             log(f"traffic {which}: not measured ({why})")
         rooflines[which] = dict(
-            bound="mfma", achieved=round(ach, 3), peak=round(MFMA_PIECES_PEAK_TFLOPS, 1),
-            unit="TFLOP/s", frac=round(ach / MFMA_PIECES_PEAK_TFLOPS, 4),
+            bound="mfma", achieved=round(ach, 3), peak=round(PROBES[which]["peak"], 1),
+            unit="TFLOP/s", frac=round(ach / PROBES[which]["peak"], 4),
             traffic=traffic["bytes"] if traffic else None,
             kernel=probe["kernel"], shape=probe["shape"], avg_launch_ms=round(probe["ms"], 5),
             launches=probe["reps"], flop_per_launch=probe["flop"],
@@ -809,6 +818,7 @@ def main():
         "sustained": sustained,
         **other_steps,
         "roofline": rooflines["fwd"],
+        "roofline_dgrad": rooflines["dgrad"],
         "roofline_wgrad": rooflines["wgrad"],
         "cpu_baseline": cpu,
         "cpu_baseline_reference_faithful": cpu_serial,
