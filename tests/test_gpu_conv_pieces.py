@@ -36,8 +36,10 @@ SHAPES = [
     (5, 20, 9, 9, 30, 5, 2),       # 5x5
     (2, 33, 27, 27, 96, 5, 2),     # 5x5 on odd planes: one LDS buffer
     (2, 16, 8, 8, 16, 5, 0),       # 5x5 without padding
-    (64, 128, 8, 8, 128, 3, 1),    # K parts as two groups of a workgroup and slices
-    (128, 96, 13, 13, 256, 3, 1),  # K slices of a grid between one and two rounds
+    (64, 128, 8, 8, 128, 3, 1),    # K slices
+    (128, 96, 13, 13, 256, 3, 1),  # a grid between one and two rounds
+    (8, 128, 28, 28, 100, 3, 1),   # two K groups of a workgroup, slices, ragged filters
+    (2, 512, 16, 16, 384, 3, 1),   # two K groups in each of 16 slices
 ]
 
 
@@ -77,7 +79,7 @@ def one_each(rng, groups, members):
 
 
 @pytest.mark.parametrize("shape", [SHAPES[1], SHAPES[3], SHAPES[4], SHAPES[5], SHAPES[12],
-                                   SHAPES[14], SHAPES[15], (128, 64, 13, 13, 320, 3, 1)],
+                                   SHAPES[14], SHAPES[16], SHAPES[17]],
                          ids=lambda s: "x".join(map(str, s)))
 def test_single_products(gpu, shape):
     """Filters with one nonzero weight for each output (and, for the input

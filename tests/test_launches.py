@@ -26,6 +26,15 @@ def test_lds_limits_do_not_depend_on_the_layer(tmp_path):
     assert all(len(v) == 1 for v in limits.values())
 
 
+def test_two_k_groups_are_tested(tmp_path):
+    """The shapes that stand for workgroups of two K groups still run them."""
+    calls = [["ach_conv_fwd", [{"conv": s}, "p", "p", "p", "p", WS, None]]
+             for s in ((8, 128, 28, 28, 100, 3, 1, 1), (2, 512, 16, 16, 384, 3, 1, 1))]
+    for r in record(calls, tmp_path):
+        assert any(v["block"][0] == 512 and v["lds"] > 0 and v["grid"][1] > 1
+                   for v in r["launches"])
+
+
 def test_batchnorm_of_many_channels(tmp_path):
     """One workgroup per channel and one launch only where they are few: a
     fully connected layer's thousands of features of a few values take the
