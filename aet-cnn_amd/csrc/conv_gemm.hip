@@ -990,9 +990,11 @@ struct FwdProblem {
 // infinite or NaN weight included (as a product with a zero it would add a
 // NaN), and the error is that of the short sums: in one chain over filters and
 // taps it was 1.3 to 2.5 times larger (32 -> 64 channels 5x5 stride 2 at 64x64,
-// batch 16: 3.7e-7 instead of 1.5e-7 from 64 bits).
+// batch 16: 3.7e-7 instead of 1.5e-7 from 64 bits).  Up to 15 filters pad to
+// 16: 11 of them, 129 channels 5x5 at 23x19, batch 53, take 41 us, 34 in one
+// chain and 1430 by image.
 // Bound: fp32 MFMA and the launch.  It replaces a GEMM and a col2im launch
-// per image: 72 -> 48 channels at 37x29, stride 2, batch 16: the layer's training pass 461 -> 90 us.
+// per image: 72 -> 48 channels at 37x29, stride 2, batch 16: 394 -> 25 us.
 constexpr int PH_MAX_S = 4;
 constexpr int PH_BK = 16;  // k-tile; a tap's filters are padded to a multiple
 struct Phase {

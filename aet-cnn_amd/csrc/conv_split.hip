@@ -34,10 +34,10 @@
 //
 // Bound: the matrix pipe at the clock that six bf16 passes sustain.  The same
 // loop without loads, splits and LDS runs 276 TFLOP/s (fp32-equivalent),
-// the kernel 215-222 where the fp32 kernel ran 141 (3x3, batch 128: 128 ->
-// 128 @ 32x32 273 -> 178 us, 384 -> 384 @ 13x13 417 -> 264 us), and 215-230
-// against 132 on 5x5 filters (96 -> 256 @ 27x27 868 -> 500 us); without the
-// filter loads 157, without LDS reads 162 of the 178 us.
+// the kernel 221-222 where the fp32 kernel ran 138-142 (3x3, batch 128: 128 ->
+// 128 @ 32x32 272 -> 175 us, 384 -> 384 @ 13x13 416 -> 259 us), and 214-233
+// against 131 on 5x5 filters (96 -> 256 @ 27x27 872 -> 493 us); without the
+// filter loads and without LDS reads 12% and 9% less.
 #include "conv_split.hpp"
 #include "pieces.hpp"
 

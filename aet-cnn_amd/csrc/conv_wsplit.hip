@@ -22,18 +22,19 @@
 // segment of one row, loaded a step ahead, split beside the MFMAs); dy rows
 // outside the image are read from a row of zeros, so a step has no branch.
 //
-// Bound: the matrix pipe beside the staging; 2.4 us per step of 54 MFMAs on
-// each of two waves per SIMD (1.44 us at the full clock).  Measured with the
-// reduction, batch 128, fp32 kernel before -> now: 128 -> 128 @ 32x32 293 ->
-// 189 us (205 TFLOP/s), 512 -> 512 @ 8x8 295 -> 187, 384 -> 384 @ 13x13 477
-// -> 325 (rows of 13 of 16 positions); batch 32, 512 -> 512 @ 8x8 88 -> 69.
+// Bound: the matrix pipe beside the staging and the additions; 2.3 us per step
+// of 54 MFMAs on each of two waves per SIMD (1.44 us at the full clock).
+// Measured with the reduction, batch 128, fp32 kernel before -> now: 128 -> 128 @
+// 32x32 286 -> 184 us (210 TFLOP/s), 512 -> 512 @ 8x8 292 -> 184, 384 -> 384 @
+// 13x13 461 -> 336 (rows of 13 of 16 positions); batch 32, 512 -> 512 @ 8x8 86 ->
+// 64.
 // Non-finite sums are computed again as in conv_split.hip: with NaNs
 // everywhere the first of these takes 920 us (310 on the fp32 kernel).  What
 // the recomputation keeps in registers is counted beside the loop's: written
 // with indexed sums it made the kernel spill 82 registers after the loop
 // (188 us instead of 183, 62.9 MB written a launch instead of 37.7).
 // Error against 64 bits, batch 128: 128 -> 128 @ 32x32 2.5e-7 (fp32 kernel
-// 8.2e-7; 7.7e-7 with one accumulator for all products, which took 183 us),
+// 8.2e-7; 7.7e-7 with one accumulator for all products, 5% faster),
 // 384 -> 384 @ 13x13 3.1e-7 (7.8e-7; 7.2e-7), batch 8, 64 -> 64 @ 112x112
 // 1.9e-7 (2.5e-7; 3.8e-7).
 // Partial sums laid out [tap][f][c], 32 channels a line: stored as dw is

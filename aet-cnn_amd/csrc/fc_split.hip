@@ -13,8 +13,8 @@
 // Bound: memory in the weight gradient (reads and writes dw: 302 MB of the
 // 9216 x 4096 layer), the split's VALU work and the latency of one chunk at
 // a time elsewhere.  Batch 128, fp32 kernels before -> now: 9216 -> 4096
-// forward 99 -> 63 us, input gradient 159 -> 68, weight gradient 130 -> 116;
-// 4096 -> 4096 56 -> 36, 53 -> 38, 88 -> 52; error against 64 bits 0.4 of
+// forward 105 -> 65 us, input gradient 161 -> 70, weight gradient 128 -> 124;
+// 4096 -> 4096 55 -> 37, 52 -> 39, 86 -> 55; error against 64 bits 0.33-0.43 of
 // theirs.  Up to 32 rows a tile is mostly padding and the fp32 kernels stay;
 // so do they for weight gradients of at most 64 images (48, 4096 -> 4096: 38
 // against 47 us) or fewer than 512 tiles.
