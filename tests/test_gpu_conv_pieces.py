@@ -646,3 +646,85 @@ def test_fully_connected_non_finite(gpu):
     assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
     fin = np.isfinite(ref)
     assert np.all(abs(got[fin] - ref[fin]) <= 1e-5 * abs(ref[fin]).max())
+
+
+def float_aligned(a):
+    """A device copy of a whose address is a multiple of 4 bytes only, and
+    what keeps it allocated."""
+    base = D(a.size + 5)
+    v = D.wrap(base.ptr + 4, a.shape)
+    v.upload(a)
+    return v, base
+
+
+@pytest.mark.parametrize("dims", [
+    (32, 256, 8, 8, 256, 3, 1, 1),   # 16-byte loads of whole segments, slices
+    (2, 64, 16, 16, 130, 3, 1, 1),
+    (4, 64, 20, 40, 64, 5, 1, 2),
+    (16, 48, 13, 13, 72, 3, 2, 1),   # by phases, float4 filter loads
+    (70, 512, 1, 1, 256, 1, 1, 0),   # fully connected, row-major 16-byte loads
+    (70, 2904, 1, 1, 2896, 1, 1, 0),
+], ids=lambda s: "x".join(map(str, s)))
+def test_addresses_of_floats(gpu, dims):
+    """Tensors at addresses that are a float's multiple only: the same bits."""
+    B, Cc, H, W, F, k, s, p = dims
+    rng = np.random.default_rng(sum(dims))
+    oh, ow = (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+    host = [rng.standard_normal(v).astype(np.float32)
+            for v in ((B, Cc, H, W), (F, Cc, k, k), (B, F, oh, ow))]
+    d = aetcnn.ConvDesc(*dims)
+    r = C.byref(d)
+    nb = max(gpu.ach_conv_fwd_workspace(r), gpu.ach_conv_bwd_data_workspace(r),
+             gpu.ach_conv_bwd_filter_workspace(r))
+    ws = D(nb // 4 + 64)
+    got = []
+    for put in (lambda a: (D.from_numpy(a), None), float_aligned):
+        bufs = [put(a) for a in host + [np.zeros_like(a) for a in host]]
+        x, w, dy, dx, dw, y = (b[0] for b in bufs)
+        check(gpu.ach_conv_fwd(r, x.ptr, w.ptr, y.ptr, ws.ptr, nb, None))
+        check(gpu.ach_conv_bwd_data(r, dy.ptr, w.ptr, dx.ptr, ws.ptr, nb, None))
+        check(gpu.ach_conv_bwd_filter(r, x.ptr, dy.ptr, dw.ptr, ws.ptr, nb, None))
+        got.append([a.numpy().view(np.uint32) for a in (y, dx, dw)])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("dims", [
+    (8, 128, 28, 28, 100, 3, 1, 1), (2, 512, 16, 16, 384, 3, 1, 1), (2, 64, 16, 16, 130, 3, 1, 1),
+    (8, 96, 20, 40, 128, 5, 1, 2), (32, 256, 8, 8, 256, 3, 1, 1), (10, 349, 20, 21, 463, 3, 1, 1),
+    (1, 36, 11, 10, 195, 5, 2, 2), (16, 48, 13, 13, 72, 3, 2, 1), (130, 520, 1, 1, 256, 1, 1, 0),
+], ids=lambda s: "x".join(map(str, s)))
+def test_workspace_limits(gpu, dims):
+    """Any workspace is refused or enough: nothing is written beyond it, and
+    the result is that of the queried size to rounding."""
+    B, Cc, H, W, F, k, s, p = dims
+    rng = np.random.default_rng(sum(dims))
+    oh, ow = (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+    x, w, dy = (D.from_numpy(rng.standard_normal(v).astype(np.float32))
+                for v in ((B, Cc, H, W), (F, Cc, k, k), (B, F, oh, ow)))
+    d = aetcnn.ConvDesc(*dims)
+    r = C.byref(d)
+    out = {"fwd": D(dy.shape), "data": D(x.shape), "filter": D(w.shape)}
+    query = {"fwd": gpu.ach_conv_fwd_workspace(r), "data": gpu.ach_conv_bwd_data_workspace(r),
+             "filter": gpu.ach_conv_bwd_filter_workspace(r)}
+    guard = np.full(1 << 16, 123.0, np.float32)
+    for op, n in query.items():
+        ref, ran = None, 0
+        for nb in sorted({n, n - 4, n * 3 // 4, n // 2, n // 3, n // 5, n // 9, n // 20} - {-4},
+                         reverse=True):
+            nb = nb // 4 * 4
+            ws = D(nb // 4 + guard.size)
+            D.wrap(ws.ptr + nb, guard.shape).upload(guard)
+            out[op].zero()
+            a = {"fwd": (x.ptr, w.ptr), "data": (dy.ptr, w.ptr), "filter": (x.ptr, dy.ptr)}[op]
+            f = {"fwd": gpu.ach_conv_fwd, "data": gpu.ach_conv_bwd_data,
+                 "filter": gpu.ach_conv_bwd_filter}[op]
+            rc = f(r, *a, out[op].ptr, ws.ptr, nb, None)
+            assert rc in (aetcnn.ACH_OK, aetcnn.ACH_EWORKSPACE) and (rc == 0 or nb < n)
+            got = out[op].numpy().astype(np.float64)
+            assert np.array_equal(D.wrap(ws.ptr + nb, guard.shape).numpy(), guard), (op, nb)
+            if rc == 0:
+                ran += 1
+                ref = got if ref is None else ref
+                assert np.linalg.norm(got - ref) <= 3e-6 * np.linalg.norm(ref), (op, nb)
+        assert ran
